@@ -1,7 +1,7 @@
 // Training and inference kernels of the learned eddy-viscosity closure's
 // network (dh_mlp_dev.h): operand packing, batched inference, the forward
-// and backward pass of a batch, the weight gradients as BF16 MFMA GEMMs
-// over the batch, the reduction of per-block partial gradients, and Adam.
+// and backward pass of a batch with the weight gradients as BF16 MFMA GEMMs
+// over its samples, the reduction of per-block partial gradients, and Adam.
 // No counterpart in the reference (its LES has no learned model).
 #include <hip/hip_runtime.h>
 
@@ -90,231 +90,267 @@ __global__ void __launch_bounds__(256) k_mlp_infer(const bf16x8 *__restrict__ pk
   }
 }
 
-// Forward and backward pass of a batch.  Loss: sum_n (softplus(y_n) -
-// t_n)^2 / N.  Writes, as BF16 rows of N samples, the layer inputs H0
-// (features, 8 rows), H1, H2, H3, the output gradient dL/dy (1 row) and the
-// pre-activation gradients dZ1, dZ2, dZ3, for the weight-gradient GEMMs,
-// and per wave the partial sum of the loss.
-__global__ void __launch_bounds__(64) k_mlp_fwd_bwd(const bf16x8 *pk, const float *P, const float *__restrict__ x,
-                                                  const float *__restrict__ t, long long N, float inv_n,
-                                                  __bf16 *__restrict__ act, float *__restrict__ part) {
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  // rows: H0 [8][N], H1..H3 [64][N], DY [8][N] (row 0 used), dZ1..dZ3 [64][N]
-  __bf16 *H0 = act, *H1 = H0 + 8 * N, *H2 = H1 + 64 * N, *H3 = H2 + 64 * N;
-  __bf16 *DY = H3 + 64 * N, *D1 = DY + 8 * N, *D2 = D1 + 64 * N, *D3 = D2 + 64 * N;
+// Loss, forward and backward pass and the weight gradients of a batch, one
+// launch.  Loss: sum_n (softplus(y_n) - t_n)^2 / N.  A block of four waves
+// takes 64 samples at a time, 16 per wave through the network and back; the
+// layer inputs H0 (features), H1..H3, dL/dy and the pre-activation gradients
+// dZ1..dZ3 go to LDS as BF16 rows of the tile's samples, which is the
+// transpose the gradient products need: 16x16x32 BF16 MFMAs with the samples
+// as K (lane l reads 8 consecutive samples of one row for A and for B),
+//   dW[in][out] = sum_n Hin[in][n] dZ[out][n],  wave w the columns
+//   out = 16 w + l % 16 of every layer (layer 1 has one row tile, inputs
+//   0..15, of which 0..7 are non-zero), the bias gradients sum_n dZ[out][n]
+//   from an A operand of ones, dW4[u] = sum_n H3[u][n] dy[n] for the rows
+//   16 w + l % 16 (dy in column 0 of B) and db4 = sum_n dy[n] (wave 0).
+// A block keeps its sums in registers over its tiles and writes them once,
+// in the parameter vector's layout, to part[block][kPartLd] (rows 8..31 of
+// W1, which have no inputs, are left out; the block's loss at kMlpNP).
+//
+// What bounds it: the chain of layers (MFMA, GELU, conversion, next MFMA) at
+// two waves per SIMD; 800 B of activations per sample stay in LDS.  With the
+// activations in device memory between a pass kernel and a product kernel of
+// one wave per 1024 samples and layer (64 waves at 16384 samples), a step of
+// 16384 samples took 100 us, 47 of them in the products and 23 in the sum
+// over 512 partial losses by one thread; this way the whole step (this
+// launch, the sum over blocks 4.5 us, the update 2.4 us) takes 21 us.
+constexpr int kTrThreads = 256, kTrTile = 64;
+constexpr int kTrLd = kTrTile + 8;      // row stride in LDS (BF16 values): rows start on different banks
+constexpr int kRH0 = 0, kRH1 = 8, kRD1 = kRH1 + 3 * kMlpH, kRDY = kRD1 + 3 * kMlpH, kTrRows = kRDY + 1;
+constexpr int kPartLd = (kMlpNP + 1 + 3) / 4 * 4;  // floats per block of partial sums
+
+__global__ void __launch_bounds__(kTrThreads, 2) k_mlp_train(const bf16x8 *pk, const float *P,
+                                                           const float *__restrict__ x, const float *__restrict__ t,
+                                                           long long N, float inv_n, float *__restrict__ part) {
+  __shared__ __bf16 act[kTrRows * kTrLd];
+  __shared__ float wloss[kTrThreads / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 aw1 = zero, aw2[4], aw3[4], ab[3], aw4 = zero, ab4 = zero;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) aw2[i] = aw3[i] = zero;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) ab[i] = zero;
+  bf16x8 ones, none;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    ones[j] = (__bf16)1.0f;
+    none[j] = (__bf16)0.0f;
+  }
   float sloss = 0.f;
-  const long long nt = (N + 15) / 16;
+  const float b4 = P[kOB4];
+  const int col = 16 * w + c;  // this lane's sample in the tile
+  const long long nt = (N + kTrTile - 1) / kTrTile;
   for (long long tile = blockIdx.x; tile < nt; tile += gridDim.x) {
-    asm volatile("" ::: "memory");  // operands re-read each pass, not held across it
-    const long long n = tile * 16 + c;
+    // operands re-read each pass: neither they nor their addresses (two
+    // registers each) are held across it
+    const bf16x8 *pl = pk + lane;
+    asm volatile("" : "+v"(pl)::"memory");
+    const long long n = tile * kTrTile + col;
     const bool live = n < N;
     const bf16x8 xb = load_x(x, N, n, N, kMlpIn);
-    f32x4 z1[4], z2[4], z3[4];
-    const float y = mlp_forward(pk, P[kOB4], xb, z1, z2, z3);
-    float dy = 0.f;
-    if (lane < 16 && live) {
-      const float r = softplus(y) - t[n];
-      sloss += r * r;
-      dy = 2.0f * r * sigmoid(y) * inv_n;
-      DY[n] = (__bf16)dy;
-    }
-    const float dys = __shfl(dy, c);  // this lane's sample
-    // 32-bit row offsets (N < 2^24 is checked by the host): every array's
-    // rows share them
-    const int Ni = (int)N, ni = (int)n;
-    if (g == 0 && live) {
+    auto put = [&](int row0, int u, float v) { act[(row0 + u) * kTrLd + col] = (__bf16)v; };
+    if (g == 0) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) H0[j * Ni + ni] = xb[j];
+      for (int j = 0; j < 8; ++j) act[(kRH0 + j) * kTrLd + col] = xb[j];
     }
-    // layer inputs (BF16, as the forward pass used them) and dZ3 = dy w4 GELU'(Z3)
-    // (w4 rounded as the forward pass used it)
-    const f32x4 *w4p = reinterpret_cast<const f32x4 *>(pk) + kPW4;
-    f32x4 d3[4];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      const f32x4 w4 = w4p[mt * 64 + lane];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int u = 16 * mt + 4 * g + i;
-        if (live) {
-          H1[u * Ni + ni] = (__bf16)gelu(z1[mt][i]);
-          H2[u * Ni + ni] = (__bf16)gelu(z2[mt][i]);
-          H3[u * Ni + ni] = (__bf16)gelu(z3[mt][i]);
-        }
-        d3[mt][i] = dys * w4[i] * gelu_grad(z3[mt][i]);
-      }
-    }
-    if (live) {
+    // forward, layer by layer; of a layer only GELU'(Z) stays in registers
+    // (its GELU(Z) in LDS, and as the next layer's operand)
+    f32x4 gp[3][4], h[4];
+    auto activate = [&](f32x4 (&z)[4], int layer) {
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) D3[(16 * mt + 4 * g + i) * Ni + ni] = (__bf16)d3[mt][i];
+        for (int i = 0; i < 4; ++i) {
+          const float zi = z[mt][i], s = gelu_s(zi);
+          h[mt][i] = zi * s;
+          gp[layer][mt][i] = gelu_grad(zi, s);
+          put(kRH1 + layer * kMlpH, 16 * mt + 4 * g + i, h[mt][i]);
+        }
+      // a layer's operands are not loaded ahead of the layer before it: all
+      // 34 together with the sums would spill
+      asm volatile("" ::: "memory");
+    };
+    const f32x4 *pb = reinterpret_cast<const f32x4 *>(pl) + kPBias;
+    {
+      const bf16x8 b[1] = {xb};
+      f32x4 z[4];
+      mlp_layer<1>(pl + kPA1, b, pb, z);
+      activate(z, 0);
     }
+#pragma unroll
+    for (int layer = 1; layer < 3; ++layer) {
+      const bf16x8 b[2] = {pack_b(h, 0), pack_b(h, 1)};
+      f32x4 z[4];
+      mlp_layer<2>(pl + (layer == 1 ? kPA2 : kPA3), b, pb + 4 * layer * 64, z);
+      activate(z, layer);
+    }
+    f32x4 yd = zero;
+    yd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[kPA4], pack_b(h, 0), yd, 0, 0, 0);
+    yd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[kPA4 + 64], pack_b(h, 1), yd, 0, 0, 0);
+    const float y = yd[0] + b4;
+    asm volatile("" ::: "memory");  // nor the backward operands
+    float dy = 0.f;  // zero for samples beyond N, and with it every gradient of theirs
+    if (lane < 16) {
+      if (live) {
+        const float r = softplus(y) - t[n];
+        sloss += r * r;
+        dy = 2.0f * r * sigmoid(y) * inv_n;
+      }
+      act[kRDY * kTrLd + col] = (__bf16)dy;
+    }
+    const float dys = __shfl(dy, c);  // this lane's sample
+    // dZ3 = dy w4 GELU'(Z3) (w4 rounded as the forward pass used it), then
     // dH2 = W3 dZ3^T, dZ2 = dH2 GELU'(Z2); dH1 = W2 dZ2^T, dZ1 = dH1 GELU'(Z1)
-    f32x4 d2[4], d1[4];
-    {
-      const bf16x8 b[2] = {pack_b(d3, 0), pack_b(d3, 1)};
+    f32x4 d[4];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      const f32x4 w4 = reinterpret_cast<const f32x4 *>(pl)[kPW4 + mt * 64];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        d[mt][i] = dys * w4[i] * gp[2][mt][i];
+        put(kRD1 + 2 * kMlpH, 16 * mt + 4 * g + i, d[mt][i]);
+      }
+    }
+#pragma unroll
+    for (int layer = 1; layer >= 0; --layer) {
+      asm volatile("" ::: "memory");
+      const bf16x8 b[2] = {pack_b(d, 0), pack_b(d, 1)};
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt) {
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
+        f32x4 q = zero;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
-          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pk[kPB3 + (mt * 2 + kb) * 64 + lane], b[kb], d, 0, 0, 0);
+          q = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[(layer ? kPB3 : kPB2) + (mt * 2 + kb) * 64], b[kb], q, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          d2[mt][i] = d[i] * gelu_grad(z2[mt][i]);
-          if (live) D2[(16 * mt + 4 * g + i) * Ni + ni] = (__bf16)d2[mt][i];
+          d[mt][i] = q[i] * gp[layer][mt][i];
+          put(kRD1 + layer * kMlpH, 16 * mt + 4 * g + i, d[mt][i]);
         }
       }
     }
-    {
-      const bf16x8 b[2] = {pack_b(d2, 0), pack_b(d2, 1)};
+    __syncthreads();
+    auto row = [&](int r, int k0) { return *reinterpret_cast<const bf16x8 *>(&act[r * kTrLd + k0 + 8 * g]); };
+#pragma unroll 1
+    for (int k0 = 0; k0 < kTrTile; k0 += 32) {
+      const bf16x8 d1b = row(kRD1 + col, k0), d2b = row(kRD1 + kMlpH + col, k0), d3b = row(kRD1 + 2 * kMlpH + col, k0);
+      const bf16x8 dyb = (c == 0) ? row(kRDY, k0) : none;
+      const bf16x8 h0 = (c < 8) ? row(kRH0 + c, k0) : none;
+      aw1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h0, d1b, aw1, 0, 0, 0);
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt) {
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pk[kPB2 + (mt * 2 + kb) * 64 + lane], b[kb], d, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          d1[mt][i] = d[i] * gelu_grad(z1[mt][i]);
-          if (live) D1[(16 * mt + 4 * g + i) * Ni + ni] = (__bf16)d1[mt][i];
-        }
+        aw2[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row(kRH1 + 16 * mt + c, k0), d2b, aw2[mt], 0, 0, 0);
+        aw3[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row(kRH1 + kMlpH + 16 * mt + c, k0), d3b, aw3[mt], 0, 0, 0);
       }
+      ab[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, d1b, ab[0], 0, 0, 0);
+      ab[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, d2b, ab[1], 0, 0, 0);
+      ab[2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, d3b, ab[2], 0, 0, 0);
+      aw4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row(kRH1 + 2 * kMlpH + col, k0), dyb, aw4, 0, 0, 0);
+      if (w == 0) ab4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, dyb, ab4, 0, 0, 0);
     }
+    __syncthreads();  // the next tile's rows go over these
   }
+  // result tiles: lane l holds rows 4 g + i of column c
+  float *o = part + (long long)blockIdx.x * kPartLd;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) sloss += __shfl_xor(sloss, o);
-  if (lane == 0) part[blockIdx.x] = sloss * inv_n;  // the loss is the mean over the batch
+  for (int i = 0; i < 4; ++i) {
+    if (g < 2) o[kOW1 + (4 * g + i) * kMlpH + col] = aw1[i];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      o[kOW2 + (16 * mt + 4 * g + i) * kMlpH + col] = aw2[mt][i];
+      o[kOW3 + (16 * mt + 4 * g + i) * kMlpH + col] = aw3[mt][i];
+    }
+    if (c == 0) o[kOW4 + 16 * w + 4 * g + i] = aw4[i];
+  }
+  if (g == 0) {  // every row of a ones tile holds the column sums
+    o[kOB1 + col] = ab[0][0];
+    o[kOB2 + col] = ab[1][0];
+    o[kOB3 + col] = ab[2][0];
+  }
+  if (threadIdx.x == 0) o[kOB4] = ab4[0];
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) sloss += __shfl_xor(sloss, s);
+  if (lane == 0) wloss[w] = sloss * inv_n;  // the loss is the mean over the batch
+  __syncthreads();
+  if (threadIdx.x == 0) o[kMlpNP] = (wloss[0] + wloss[1]) + (wloss[2] + wloss[3]);
 }
 
-// Parameter gradients of layer L = blockIdx.y over the samples of slice
-// blockIdx.x, as 16x16x32 BF16 MFMAs with the samples as K (lane l reads 8
-// consecutive samples of one row for A and for B):
-//   L = 0..2: dW[in][out] = sum_n Hin[in][n] dZ[out][n] (A rows in =
-//             16 mt + l % 16, B rows out = 16 nt + l % 16; layer 0 has one
-//             row tile, inputs 0..15, of which 0..7 are stored), and the
-//             bias gradient sum_n dZ[out][n] from an A operand of ones;
-//   L = 3:    dW4[u] = sum_n H3[u][n] dy[n] and db4 = sum_n dy[n] (B = the
-//             dy row in column 0).
-// Partial sums to wpart[slice][L][65][64]: rows 0..63 the weights (dW4 in
-// column 0), row 64 the bias.
-constexpr int kWRows = 65;
-
-__global__ void __launch_bounds__(64) k_mlp_wgrad(const __bf16 *__restrict__ act, long long N, long long per_slice,
-                                                float *__restrict__ wpart) {
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const int layer = blockIdx.y;
-  const __bf16 *H0 = act, *H1 = H0 + 8 * N, *H2 = H1 + 64 * N, *H3 = H2 + 64 * N;
-  const __bf16 *DY = H3 + 64 * N, *D1 = DY + 8 * N, *D2 = D1 + 64 * N, *D3 = D2 + 64 * N;
-  const __bf16 *Hin = (layer == 0) ? H0 : (layer == 1) ? H1 : (layer == 2) ? H2 : H3;
-  const __bf16 *Dz = (layer == 0) ? D1 : (layer == 1) ? D2 : (layer == 2) ? D3 : DY;
-  const int mts = (layer == 0) ? 1 : 4, nts = (layer == 3) ? 1 : 4;
-  f32x4 acc[5][4];  // row tiles 0..3 of the weights, 4: the bias (A of ones)
-#pragma unroll
-  for (int mt = 0; mt < 5; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 ones;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
-  const long long n_lo = (long long)blockIdx.x * per_slice, n_hi = min(N, n_lo + per_slice);
-  for (long long n0 = n_lo; n0 < n_hi; n0 += 32) {
-    const long long n = n0 + 8 * g;  // N is a multiple of 32: whole 8-sample groups
-    bf16x8 b[4];
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      if (nt < nts) {
-        if (layer == 3) {  // column 0: dy; the others zero
-          if (c == 0) {
-            b[nt] = *reinterpret_cast<const bf16x8 *>(Dz + n);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) b[nt][j] = (__bf16)0.0f;
-          }
-        } else {
-          b[nt] = *reinterpret_cast<const bf16x8 *>(Dz + (16 * nt + c) * N + n);
-        }
-      }
-    }
-#pragma unroll
-    for (int mt = 0; mt < 5; ++mt) {
-      if (mt < 4 && mt >= mts) continue;
-      bf16x8 a;
-      if (mt == 4) {
-        a = ones;
-      } else if (layer == 0) {
-        if (c < 8) {
-          a = *reinterpret_cast<const bf16x8 *>(Hin + c * N + n);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) a[j] = (__bf16)0.0f;
-        }
-      } else {
-        a = *reinterpret_cast<const bf16x8 *>(Hin + (16 * mt + c) * N + n);
-      }
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
-        if (nt < nts) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[nt], acc[mt][nt], 0, 0, 0);
-    }
-  }
-  float *o = wpart + ((long long)blockIdx.x * 4 + layer) * (kWRows * kMlpH);
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    if (mt >= mts) continue;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-      if (nt < nts)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[(16 * mt + 4 * g + i) * kMlpH + 16 * nt + c] = acc[mt][nt][i];
-  }
-  // the bias row: every row of the ones tile holds the column sums; take row 0
-  if (g == 0) {
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-      if (nt < nts) o[64 * kMlpH + 16 * nt + c] = acc[4][nt][0];
-  }
-}
-
-// grad[p] = the sum over slices of the partial sums, in the parameter
-// vector's layout (W1 rows 8..31 are zero: their inputs are zero); loss =
-// the sum over waves of their parts of the batch mean.
-__global__ void k_mlp_reduce(const float *__restrict__ wpart, int nslice, const float *__restrict__ part, int nwave,
-                             float *__restrict__ grad, float *__restrict__ loss) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > kMlpNP) return;
-  if (p == kMlpNP) {
-    float a = 0.f;
-    for (int k = 0; k < nwave; ++k) a += part[k];
-    *loss = a;
-    return;
-  }
-  int layer, row, col;
-  if (p < kOB1) { layer = 0; row = (p - kOW1) / kMlpH; col = (p - kOW1) % kMlpH; }
-  else if (p < kOW2) { layer = 0; row = 64; col = p - kOB1; }
-  else if (p < kOB2) { layer = 1; row = (p - kOW2) / kMlpH; col = (p - kOW2) % kMlpH; }
-  else if (p < kOW3) { layer = 1; row = 64; col = p - kOB2; }
-  else if (p < kOB3) { layer = 2; row = (p - kOW3) / kMlpH; col = (p - kOW3) % kMlpH; }
-  else if (p < kOW4) { layer = 2; row = 64; col = p - kOB3; }
-  else if (p < kOB4) { layer = 3; row = p - kOW4; col = 0; }
-  else { layer = 3; row = 64; col = 0; }
+// grad[p] = the sum of the blocks' partial sums (rows 8..31 of W1 are zero:
+// their inputs are zero); loss = the sum of their parts of the batch mean.
+// A block takes 64 values, its four waves every fourth partial sum each, so
+// that 165 blocks of four waves read the partial sums (42 KB per block of
+// k_mlp_train) with eight loads in flight per lane.
+__global__ void __launch_bounds__(256) k_mlp_reduce(const float *__restrict__ part, int nblk, float *__restrict__ grad,
+                                                  float *__restrict__ loss) {
+  __shared__ float sm[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, p = blockIdx.x * 64 + lane;
+  const bool padding = p >= 8 * kMlpH && p < kOB1;
   float a = 0.f;
-  if (!(layer == 0 && row >= 16 && row < 64))
-    for (int k = 0; k < nslice; ++k) a += wpart[((long long)k * 4 + layer) * (kWRows * kMlpH) + row * kMlpH + col];
-  grad[p] = a;
+  if (p <= kMlpNP && !padding) {
+#pragma unroll 8
+    for (int k = w; k < nblk; k += 4) a += part[(long long)k * kPartLd + p];
+  }
+  sm[w][lane] = a;
+  __syncthreads();
+  if (w != 0 || p > kMlpNP) return;
+  a = (sm[0][lane] + sm[1][lane]) + (sm[2][lane] + sm[3][lane]);
+  if (p == kMlpNP)
+    *loss = a;
+  else
+    grad[p] = a;
 }
 
 // Adam (Kingma & Ba 2015) on the FP32 parameters; c1 = 1 - beta1^t,
-// c2 = 1 - beta2^t come from the host
-__global__ void k_mlp_adam(float *__restrict__ P, float *__restrict__ m, float *__restrict__ v,
-                           const float *__restrict__ grad, float lr, float b1, float b2, float eps, float c1, float c2) {
+// c2 = 1 - beta2^t come from the host.  Each thread also writes its new
+// parameter to every place k_mlp_pack would put it (the zero rows of the
+// output layer's operand included), so the update is one launch; a second
+// one for the packing took 4.8 us and the gap before it, at 5 us a launch
+// for 42 KB of parameters.
+__global__ void __launch_bounds__(64) k_mlp_adam_pack(float *__restrict__ P, float *__restrict__ m,
+                                                    float *__restrict__ v, const float *__restrict__ grad, float lr,
+                                                    float b1, float b2, float eps, float c1, float c2,
+                                                    bf16x8 *__restrict__ pk) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= kMlpNP) return;
   const float gr = grad[p];
   const float mm = b1 * m[p] + (1.f - b1) * gr, vv = b2 * v[p] + (1.f - b2) * gr * gr;
   m[p] = mm;
   v[p] = vv;
-  P[p] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+  const float w = P[p] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+  P[p] = w;
+  __bf16 *q = reinterpret_cast<__bf16 *>(pk);
+  float *qf = reinterpret_cast<float *>(pk);
+  const __bf16 wb = (__bf16)w;
+  // lane and element of unit u (mlp_unit's inverse): K block u / 32, lane
+  // group (u / 4) % 4, element 4 ((u / 16) % 2) + u % 4
+  auto unit = [](int u, int c) { return ((u >> 5) * 64 + 16 * ((u >> 2) & 3) + c) * 8 + 4 * ((u >> 4) & 1) + (u & 3); };
+  auto tile = [&](int base, int u, float val) {  // result-tile layout, the 16 lanes of the unit's group
+#pragma unroll
+    for (int c = 0; c < 16; ++c) qf[(base + (u >> 4) * 64 + 16 * ((u >> 2) & 3) + c) * 4 + (u & 3)] = val;
+  };
+  auto hidden = [&](int pa, int pb, int r) {  // W[in][out] as A (transposed) and B operands
+    const int in = r / kMlpH, out = r % kMlpH;
+    q[(pa + (out >> 4) * 128) * 8 + unit(in, out & 15)] = wb;
+    q[(pb + (in >> 4) * 128) * 8 + unit(out, in & 15)] = wb;
+  };
+  if (p < kOB1) {
+    const int in = p / kMlpH, out = p % kMlpH;
+    q[(kPA1 + (out >> 4) * 64 + 16 * (in >> 3) + (out & 15)) * 8 + (in & 7)] = wb;
+  } else if (p < kOW2) {
+    tile(kPBias, p - kOB1, w);
+  } else if (p < kOB2) {
+    hidden(kPA2, kPB2, p - kOW2);
+  } else if (p < kOW3) {
+    tile(kPBias + 4 * 64, p - kOB2, w);
+  } else if (p < kOB3) {
+    hidden(kPA3, kPB3, p - kOW3);
+  } else if (p < kOW4) {
+    tile(kPBias + 8 * 64, p - kOB3, w);
+  } else if (p < kOB4) {
+    const int u = p - kOW4;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) q[kPA4 * 8 + unit(u, c)] = c == 0 ? wb : (__bf16)0.0f;
+    tile(kPW4, u, (float)wb);
+  }
 }
 
 hipError_t launch_mlp_pack(const float *params, void *packed, hipStream_t st) {
@@ -332,13 +368,10 @@ int mlp_fail(int code, const std::string &msg) {
   g_mlp_err = msg;
   return code;
 }
-constexpr int kWaves = 512;            // blocks of k_mlp_fwd_bwd (one wave each)
-constexpr long long kSliceMin = 1024;  // samples per weight-gradient slice at least
-long long n_slices(long long n) { return std::max<long long>(1, std::min<long long>(256, n / kSliceMin)); }
-long long per_slice(long long n) {
-  const long long s = n_slices(n);
-  return ((n + s - 1) / s + 31) / 32 * 32;
-}
+// blocks of k_mlp_train: one per 64-sample tile up to two per CU (57 KB of
+// LDS each); more samples loop
+constexpr long long kTrBlocks = 512;
+long long train_blocks(long long n) { return std::min<long long>(kTrBlocks, (n + kTrTile - 1) / kTrTile); }
 }  // namespace
 
 extern "C" {
@@ -351,10 +384,7 @@ int64_t dh_mlp_packed_bytes(void) { return 16LL * kPAll; }
 
 int64_t dh_mlp_work_bytes(int64_t n) {
   if (n <= 0) return 0;
-  const long long act = 2LL * n * (16 + 6 * 64);
-  const long long wp = 4LL * n_slices(n) * 4 * kWRows * kMlpH;
-  const long long pp = 4LL * kWaves;
-  return act + wp + pp;
+  return 4LL * train_blocks(n) * kPartLd;
 }
 
 int dh_mlp_pack_dev(const float *params, void *packed, void *stream) {
@@ -384,16 +414,11 @@ int dh_mlp_grad_dev(const float *params, const void *packed, const float *x, con
   if (n > (1LL << 24)) return mlp_fail(DH_EARG, "the batch must hold at most 2^24 samples");
   if (work_bytes < dh_mlp_work_bytes(n)) return mlp_fail(DH_EARG, "work buffer smaller than dh_mlp_work_bytes(n)");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  char *w = static_cast<char *>(work);
-  __bf16 *act = reinterpret_cast<__bf16 *>(w);
-  float *wp = reinterpret_cast<float *>(w + 2LL * n * (16 + 6 * 64));
-  const long long ns = n_slices(n);
-  float *part = wp + ns * 4 * kWRows * kMlpH;
-  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(kWaves), dim3(64), 0, st, static_cast<const bf16x8 *>(packed), params, x,
-                     target, (long long)n, 1.0f / (float)n, act, part);
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3((unsigned)ns, 4), dim3(64), 0, st, act, (long long)n, per_slice(n), wp);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpNP + 1 + 255) / 256), dim3(256), 0, st, wp, (int)ns, part, kWaves, grad,
-                     loss);
+  float *part = static_cast<float *>(work);
+  const int nb = (int)train_blocks(n);
+  hipLaunchKernelGGL(k_mlp_train, dim3(nb), dim3(kTrThreads), 0, st, static_cast<const bf16x8 *>(packed), params, x,
+                     target, (long long)n, 1.0f / (float)n, part);
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpNP + 1 + 63) / 64), dim3(256), 0, st, part, nb, grad, loss);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? DH_OK : mlp_fail(DH_EHIP, hipGetErrorString(e));
 }
@@ -405,9 +430,8 @@ int dh_mlp_adam_dev(float *params, float *m, float *v, const float *grad, float 
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.0f - powf(b1, (float)step), c2 = 1.0f - powf(b2, (float)step);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpNP + 255) / 256), dim3(256), 0, st, params, m, v, grad, lr, b1, b2, 1e-8f,
-                     c1, c2);
-  hipLaunchKernelGGL(k_mlp_pack, dim3((kPAll + 255) / 256), dim3(256), 0, st, params, static_cast<bf16x8 *>(packed));
+  hipLaunchKernelGGL(k_mlp_adam_pack, dim3((kMlpNP + 63) / 64), dim3(64), 0, st, params, m, v, grad, lr, b1, b2, 1e-8f,
+                     c1, c2, static_cast<bf16x8 *>(packed));
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? DH_OK : mlp_fail(DH_EHIP, hipGetErrorString(e));
 }

@@ -65,9 +65,9 @@ __device__ __forceinline__ float gelu_s(float z) {
   return __builtin_amdgcn_rcpf(e + 1.0f);
 }
 __device__ __forceinline__ float gelu(float z) { return z * gelu_s(z); }
-// d GELU / dz = s + z s (1 - s) 2 a'(z), a'(z) = sqrt(2/pi) (1 + 3 0.044715 z^2)
-__device__ __forceinline__ float gelu_grad(float z) {
-  const float s = gelu_s(z);
+// d GELU / dz = s + z s (1 - s) 2 a'(z), a'(z) = sqrt(2/pi) (1 + 3 0.044715 z^2),
+// s = gelu_s(z)
+__device__ __forceinline__ float gelu_grad(float z, float s) {
   return fmaf(z * s * (1.0f - s), 1.5957691216057308f * fmaf(0.134145f, z * z, 1.0f), s);
 }
 __device__ __forceinline__ float softplus(float y) { return fmaxf(y, 0.0f) + log1pf(__expf(-fabsf(y))); }
@@ -86,57 +86,17 @@ __device__ __forceinline__ bf16x8 pack_b(const f32x4 (&h)[4], int kb) {
 }
 
 // One hidden layer: Z = W^T Hin + bias for the 4 output tiles (KB K
-// blocks); bias: the layer's packed biases (f32x4 per lane and tile).
+// blocks); A, bias: this lane's first packed operand and bias tile of the
+// layer.
 template <int KB>
 __device__ __forceinline__ void mlp_layer(const bf16x8 *A, const bf16x8 (&B)[KB], const f32x4 *bias, f32x4 (&z)[4]) {
-  const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt) {
-    f32x4 d = bias[mt * 64 + lane];
+    f32x4 d = bias[mt * 64];
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[(mt * KB + kb) * 64 + lane], B[kb], d, 0, 0, 0);
+    for (int kb = 0; kb < KB; ++kb) d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[(mt * KB + kb) * 64], B[kb], d, 0, 0, 0);
     z[mt] = d;
   }
-}
-
-// Forward pass of one 16-sample tile.  x: this lane's B operand of layer 1
-// (features 8 g + j of sample l % 16).  z1..z3: the pre-activations
-// (result-tile layout); returns the output y of sample l % 16 in lanes 0..15
-// (other lanes hold the padding rows' results).
-// b4: the output bias.
-__device__ __forceinline__ float mlp_forward(const bf16x8 *pk, float b4, const bf16x8 &x, f32x4 (&z1)[4],
-                                             f32x4 (&z2)[4], f32x4 (&z3)[4]) {
-  const int lane = threadIdx.x & 63;
-  const f32x4 *pb = reinterpret_cast<const f32x4 *>(pk) + kPBias;
-  {
-    const bf16x8 b[1] = {x};
-    mlp_layer<1>(pk + kPA1, b, pb, z1);
-  }
-  f32x4 h[4];
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) h[mt][i] = gelu(z1[mt][i]);
-  {
-    const bf16x8 b[2] = {pack_b(h, 0), pack_b(h, 1)};
-    mlp_layer<2>(pk + kPA2, b, pb + 4 * 64, z2);
-  }
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) h[mt][i] = gelu(z2[mt][i]);
-  {
-    const bf16x8 b[2] = {pack_b(h, 0), pack_b(h, 1)};
-    mlp_layer<2>(pk + kPA3, b, pb + 8 * 64, z3);
-  }
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) h[mt][i] = gelu(z3[mt][i]);
-  f32x4 d = {0.f, 0.f, 0.f, 0.f};
-  d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pk[kPA4 + lane], pack_b(h, 0), d, 0, 0, 0);
-  d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pk[kPA4 + 64 + lane], pack_b(h, 1), d, 0, 0, 0);
-  return d[0] + b4;
 }
 
 // Inference holds this lane's forward operands in registers for a wave's
@@ -156,7 +116,10 @@ __device__ __forceinline__ void mlp_load_regs(const bf16x8 *pk, MlpRegs &r) {
   for (int i = 0; i < 12; ++i) r.b[i] = pb[i * 64 + lane];
 }
 
-// mlp_forward's output y (in lanes 0..15) from the operands in registers.
+// Forward pass of one 16-sample tile from the operands in registers.  x: this
+// lane's B operand of layer 1 (features 8 g + j of sample l % 16); b4: the
+// output bias.  Returns the output y of sample l % 16 in lanes 0..15 (other
+// lanes hold the padding rows' results).
 __device__ __forceinline__ float mlp_forward_regs(const MlpRegs &r, float b4, const bf16x8 &x) {
   static_assert(kPA2 - kPA1 == 4 * 64 && kPA3 - kPA1 == 12 * 64 && kPA4 - kPA1 == 20 * 64, "A operand order");
   f32x4 z[4], h[4];
