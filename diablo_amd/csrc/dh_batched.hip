@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 
 #include "dh_fft_dev.h"
 
@@ -30,56 +31,70 @@ namespace dh {
 // the system and are dropped, as the reference's sweeps never read them.
 // Layout [row][system], systems fastest.
 //
-// A wave solves 64/SEG systems, SEG lanes each (lane = (64/SEG) p + s).
-// Lane p holds rows [R p, R p + R) of its system in registers (rows at or beyond ny are
-// identity rows with zero right-hand side, which leave the others alone) and
+// A block of four waves solves 256/SEG systems, SEG lanes each: wave w, lane
+// (256/SEG) p + s holds segment w SEG/4 + p of system s, so that a wave's
+// access to one row of each of its segments is whole cache lines (128 B per
+// segment for SEG = 32 in FP64).  A lane holds rows [R p', R p' + R) of its
+// system, p' its segment, in registers (rows at or beyond ny are identity
+// rows with zero right-hand side, which leave the others alone) and
 // eliminates them locally, Thomas on the segment with its outer couplings
 // dropped, so that
 //   x_r = y_r - v_r X_L - w_r X_R,
 // X_L, X_R the solution just outside the segment (the partition or SPIKE
 // method): y = T^-1 d, v = T^-1 a_0 e_0, w = T^-1 c_{R-1} e_{R-1}.  The first
-// and last rows of every segment give a 2 x 2 block-tridiagonal system over
-// the SEG-1 interfaces, which one lane per system solves by block elimination.
-// Each lane then sweeps its rows again with the boundary terms moved to the
-// right-hand side.  The forward-swept right-hand side, c/pivot and 1/pivot
-// stay in registers between the sweeps (4 reals per row); the spike's
-// forward values are formed again when needed.  Loads and
-// stores are the right-hand side and the solution only (the diagonals come
-// from alpha and the two row tables): 32 bytes per row in FP64.
+// and last rows of the segments give a 2 x 2 block-tridiagonal system over
+// the interfaces, reduced cyclically across the wave's segments and then
+// joined over the four waves through LDS.  Each lane then sweeps its rows
+// again with the boundary terms moved to the right-hand side.  The
+// forward-swept right-hand side, c/pivot and 1/pivot stay in registers
+// between the sweeps (4 reals per row); the spike's forward values are
+// formed again when needed.  Loads and stores are the right-hand side and
+// the solution only (the diagonals come from alpha and the row tables): 32
+// bytes per row in FP64.
+//
+// What bounds it: in FP64 memory (257 rows of 131584 systems, 1.08 GB, in
+// 0.252 ms: 4.3 TB/s, where a plain copy of that size reaches 4.9), in FP32
+// (0.197 ms, 2.8 TB/s) and below some 10^4 systems the chain of each lane's
+// sweeps.  With one lane per system for the interfaces (31 dependent
+// eliminations while 31 lanes wait) and 32 B row segments per wave it took
+// 0.481 and 0.274 ms; the cyclic reduction alone took FP64 to 0.284, row
+// tables that need no tests to 0.271, whole cache lines per wave the rest.
 // ---------------------------------------------------------------------------
 constexpr int kCnThreads = 256;
-constexpr int kCnRows = 9;       // rows per lane
+constexpr int kCnRows = 9;  // rows per lane: 36 + 36 registers of a segment in FP64, three waves per SIMD
 constexpr int kCnMaxNy = 32 * kCnRows;
+constexpr int cn_systems(int seg) { return 256 / seg; }  // systems per block
 
-// SEG segments (lanes) per system, 64 / SEG systems per wave: 16 for ny <=
-// 144, 32 for ny <= 288 (9 rows per lane either way, which keeps the FP64
-// solve within 168 registers).
+// SEG segments (lanes) per system: the fewest of 4, 8, 16, 32 whose 9 rows
+// per lane hold ny, so that short systems do not pay for identity rows (60
+// rows of 99999 systems: 44 us with 8 segments, 64 with 16; 30 rows of 90001
+// in FP32: 12 us with 4, 67 with 16 segments before).
 template <int R, int SEG, class C>
-__device__ __forceinline__ void cn_solve_wave(const double *__restrict__ alpha, const C *__restrict__ rhs,
-                                              C *__restrict__ x, int ny, long long nsys, Sc<C> *red,
-                                              const Sc<C> *sl, const Sc<C> *su) {
+__device__ __forceinline__ void cn_solve_block(const double *__restrict__ alpha, const C *__restrict__ rhs,
+                                              C *__restrict__ x, int ny, long long nsys, const Sc<C> *tab, Sc<C> *xch) {
   using S = Sc<C>;
-  constexpr int kCnSeg = SEG, kCnSys = 64 / SEG;
-  const int lane = threadIdx.x & 63;
+  constexpr int kRows = SEG * R, kCnSys = cn_systems(SEG), kCnSeg = 64 / kCnSys;  // systems and segments per wave
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int p = lane / kCnSys, sw = lane % kCnSys;
-  const long long wave = (long long)blockIdx.x * (kCnThreads / 64) + (threadIdx.x >> 6);
-  const long long sys = wave * kCnSys + sw;
+  // Workgroups are dealt to the 8 XCDs in turn: XCD x takes a contiguous range
+  // of systems, since a block's row segment is one or two whole cache lines in
+  // FP64 (half of that in FP32) only where nsys keeps it aligned, and blocks
+  // that share a line should share an L2
+  long long blk;
+  {
+    const int b = blockIdx.x, xcd = b & 7, q = (int)gridDim.x >> 3, r = (int)gridDim.x & 7;
+    blk = (long long)xcd * q + min(xcd, r) + (b >> 3);
+  }
+  const long long sys = blk * kCnSys + sw;
   const bool live = sys < nsys;
   const long long sysc = live ? sys : nsys - 1;  // loads of idle lanes stay in bounds
-  const int r0 = p * R;
+  const int r0 = (w * kCnSeg + p) * R;
   const S al = S(alpha[sysc]);
-  // row coefficients (rows beyond ny: identity; the outer couplings dropped)
+  const S *ta = tab + r0, *tc = ta + kRows, *tb = tc + kRows;
   auto coef = [&](int r, S &a, S &b, S &c) {
-    const int j = r0 + r;
-    if (j < ny) {
-      a = (j == 0) ? S(0) : -al * sl[j];
-      c = (j == ny - 1) ? S(0) : -al * su[j];
-      b = S(1) + al * (sl[j] + su[j]);
-    } else {
-      a = S(0);
-      b = S(1);
-      c = S(0);
-    }
+    a = -al * ta[r];
+    c = -al * tc[r];
+    b = S(1) + al * tb[r];
   };
 
   C d[R];
@@ -114,7 +129,9 @@ __device__ __forceinline__ void cn_solve_wave(const double *__restrict__ alpha, 
   }
   // first-row values: y_0 and w_0 by the backward recurrences (no storage),
   // v_0 = a_0 (T^-1)_00 = a_0 / q_0 with q the pivots of an elimination from
-  // the bottom: q_{R-1} = b_{R-1}, q_r = b_r - c_r a_{r+1} / q_{r+1}
+  // the bottom: q_{R-1} = b_{R-1}, q_r = b_r - c_r a_{r+1} / q_{r+1} (formed
+  // from the top's pivots instead, without these divisions, v_0 raised the
+  // FP32 solution's error by 3%)
   // (the empty asm makes every sweep read its row tables from LDS again
   // rather than keep the previous sweep's coefficients in registers)
   asm volatile("" ::: "memory");
@@ -122,90 +139,116 @@ __device__ __forceinline__ void cn_solve_wave(const double *__restrict__ alpha, 
   S wf, wl = cp[R - 1], vf, vl = vlast;
   {
     C yy = d[R - 1];
-    S ww = cp[R - 1];
+    S ww = cp[R - 1], q, anext, c;
+    coef(R - 1, anext, q, c);
 #pragma unroll
     for (int r = R - 2; r >= 0; --r) {
+      S a, b;
+      coef(r, a, b, c);
       yy = mkc<C>(d[r].x - cp[r] * yy.x, d[r].y - cp[r] * yy.y);
       ww = -cp[r] * ww;
-    }
-    yf = yy;
-    wf = ww;
-    asm volatile("" ::: "memory");
-    S an, bn, cn;
-    coef(R - 1, an, bn, cn);
-    S q = bn, anext = an;
-#pragma unroll
-    for (int r = R - 2; r >= 0; --r) {
-      S a, b, c;
-      coef(r, a, b, c);
       q = b - c * anext / q;
       anext = a;
     }
+    yf = yy;
+    wf = ww;
     vf = a0 / q;
   }
-  // the segment's first and last rows to the wave's exchange area:
-  // [sys][p][8] = y_first (2), y_last (2), v_first, v_last, w_first, w_last
-  S *rw = red + ((threadIdx.x >> 6) * kCnSys + sw) * (kCnSeg * 8);
-  {
-    S *q = rw + p * 8;
-    q[0] = yf.x; q[1] = yf.y; q[2] = yl.x; q[3] = yl.y;
-    q[4] = vf; q[5] = vl; q[6] = wf; q[7] = wl;
+  // The segments' first and last values F_p, L_p satisfy
+  //   F_p = yf - vf L_{p-s} - wf F_{p+s},   L_p = yl - vl L_{p-s} - wl F_{p+s}
+  // with s = 1.  Each step eliminates a = L_{p-s} and b = F_{p+s} with the
+  // equations of the lanes p - s (') and p + s (''):
+  //   (1 - wl' vf) a - wl' wf b   = yl' - wl' yf   - vl' L_{p-2s}
+  //   -vf'' vl a + (1 - vf'' wl) b = yf'' - vf'' yl - wf'' F_{p+2s}
+  // which doubles s.  A neighbour outside the wave's segments stays an
+  // unknown, the same one for every lane (the equations a = A, b = B: vl' =
+  // -1, wf'' = -1), so after log2(segments per wave) steps with all lanes at
+  // work F and L depend on X_l and X_r alone, the values just outside the
+  // wave's segments.
+#pragma unroll
+  for (int s = 1; s < kCnSeg; s *= 2) {
+    const int ds = kCnSys * s;
+    const bool lo = p >= s, hi = p + s < kCnSeg;
+    C yl1 = mkc<C>(__shfl_up(yl.x, ds), __shfl_up(yl.y, ds));
+    S vl1 = __shfl_up(vl, ds), wl1 = __shfl_up(wl, ds);
+    C yf2 = mkc<C>(__shfl_down(yf.x, ds), __shfl_down(yf.y, ds));
+    S vf2 = __shfl_down(vf, ds), wf2 = __shfl_down(wf, ds);
+    yl1 = mkc<C>(lo ? yl1.x : S(0), lo ? yl1.y : S(0));
+    yf2 = mkc<C>(hi ? yf2.x : S(0), hi ? yf2.y : S(0));
+    vl1 = lo ? vl1 : S(-1);
+    wl1 = lo ? wl1 : S(0);
+    vf2 = hi ? vf2 : S(0);
+    wf2 = hi ? wf2 : S(-1);
+    const S m00 = S(1) - wl1 * vf, m01 = -(wl1 * wf), m10 = -(vf2 * vl), m11 = S(1) - vf2 * wl;
+    const S id = S(1) / (m00 * m11 - m01 * m10);
+    // [a b] = (constant) - (A) L_{p-2s} - (B) F_{p+2s}
+    const C ca = mkc<C>(yl1.x - wl1 * yf.x, yl1.y - wl1 * yf.y), cb = mkc<C>(yf2.x - vf2 * yl.x, yf2.y - vf2 * yl.y);
+    const S i00 = m11 * id, i01 = -m01 * id, i10 = -m10 * id, i11 = m00 * id;
+    const C ka = mkc<C>(i00 * ca.x + i01 * cb.x, i00 * ca.y + i01 * cb.y);
+    const C kb = mkc<C>(i10 * ca.x + i11 * cb.x, i10 * ca.y + i11 * cb.y);
+    const S aA = i00 * vl1, bA = i10 * vl1, aB = i01 * wf2, bB = i11 * wf2;
+    yf = mkc<C>(yf.x - vf * ka.x - wf * kb.x, yf.y - vf * ka.y - wf * kb.y);
+    yl = mkc<C>(yl.x - vl * ka.x - wl * kb.x, yl.y - vl * ka.y - wl * kb.y);
+    const S nvf = -(vf * aA + wf * bA), nwf = -(vf * aB + wf * bB);
+    const S nvl = -(vl * aA + wl * bA), nwl = -(vl * aB + wl * bB);
+    vf = nvf;
+    wf = nwf;
+    vl = nvl;
+    wl = nwl;
   }
-  wave_lds_sync();
-  // interfaces i = 0..SEG-2: P_i = x(last row of segment i), Q_i = x(first
-  // row of segment i+1):
+  // The four waves' first and last values, joined the same way by every lane
+  // for its system: P_i = last value of wave i, Q_i = first of wave i + 1,
   //   P_i + vl_i P_{i-1} + wl_i Q_i         = yl_i
   //   vf_{i+1} P_i + Q_i + wf_{i+1} Q_{i+1} = yf_{i+1}
-  // with P_{-1} = Q_{SEG-1} = 0 (no rows outside the system).  Block elimination
-  // keeps U-hat = [[0, c0], [0, c1]] (only Q_{i+1} couples forward).
+  // with P_{-1} = Q_3 = 0 (no rows outside the system).
+  constexpr int kW = kCnThreads / 64;
   if (p == 0) {
-    // forward elimination; the eliminated coefficients of interface i go
-    // to slots the later steps no longer read: r0 -> [i][2,3], c0 -> [i][5],
-    // r1 -> [i+1][0,1], c1 -> [i+1][4]
+    S *q = xch + (w * kCnSys + sw) * 8;
+    q[0] = yf.x; q[1] = yf.y; q[2] = vf; q[3] = wf;
+  }
+  if (p == kCnSeg - 1) {
+    S *q = xch + (w * kCnSys + sw) * 8;
+    q[4] = yl.x; q[5] = yl.y; q[6] = vl; q[7] = wl;
+  }
+  __syncthreads();
+  C Xl = mkc<C>(S(0), S(0)), Xr = Xl;
+  {
+    S c0[kW - 1], c1[kW - 1];
+    C r0v[kW - 1], r1v[kW - 1];
     S pc0 = S(0);
     C prP = mkc<C>(S(0), S(0));
-#pragma unroll 1
-    for (int i = 0; i < kCnSeg - 1; ++i) {
-      S *qi = rw + i * 8, *qn = rw + (i + 1) * 8;
-      const C ylv = mkc<C>(qi[2], qi[3]), yfv = mkc<C>(qn[0], qn[1]);
-      const S vli = qi[5], wli = qi[7], vfn = qn[4], wfn = qn[6];
-      // M = [[1, wl - vl c0_{i-1}], [vf, 1]], rhs = (yl - vl rP_{i-1}, yf),
-      // M^{-1} = [[1, -m01], [-vf, 1]] / det
+#pragma unroll
+    for (int i = 0; i < kW - 1; ++i) {
+      const S *qi = xch + (i * kCnSys + sw) * 8, *qn = qi + kCnSys * 8;
+      const C ylv = mkc<C>(qi[4], qi[5]), yfv = mkc<C>(qn[0], qn[1]);
+      const S vli = qi[6], wli = qi[7], vfn = qn[2], wfn = qn[3];
       const S m01 = wli - vli * pc0;
       const S idet = S(1) / (S(1) - m01 * vfn);
       const C t0 = mkc<C>(ylv.x - vli * prP.x, ylv.y - vli * prP.y);
-      const S c0 = -m01 * wfn * idet, c1 = wfn * idet;
-      const C rr0 = mkc<C>((t0.x - m01 * yfv.x) * idet, (t0.y - m01 * yfv.y) * idet);
-      const C rr1 = mkc<C>((yfv.x - vfn * t0.x) * idet, (yfv.y - vfn * t0.y) * idet);
-      qi[2] = rr0.x; qi[3] = rr0.y; qi[5] = c0;
-      qn[0] = rr1.x; qn[1] = rr1.y; qn[4] = c1;
-      pc0 = c0;
-      prP = rr0;
+      c0[i] = -m01 * wfn * idet;
+      c1[i] = wfn * idet;
+      r0v[i] = mkc<C>((t0.x - m01 * yfv.x) * idet, (t0.y - m01 * yfv.y) * idet);
+      r1v[i] = mkc<C>((yfv.x - vfn * t0.x) * idet, (yfv.y - vfn * t0.y) * idet);
+      pc0 = c0[i];
+      prP = r0v[i];
     }
-    // back substitution u_i = r_i - (c0_i, c1_i) Q_{i+1}; X_L of segment i+1
-    // (= P_i) to [i+1][0,1], X_R of segment i (= Q_i) to [i][2,3]
     C qn = mkc<C>(S(0), S(0));
-#pragma unroll 1
-    for (int i = kCnSeg - 2; i >= 0; --i) {
-      S *qi = rw + i * 8, *qx = rw + (i + 1) * 8;
-      const C rr0 = mkc<C>(qi[2], qi[3]), rr1 = mkc<C>(qx[0], qx[1]);
-      const S c0 = qi[5], c1 = qx[4];
-      const C P = mkc<C>(rr0.x - c0 * qn.x, rr0.y - c0 * qn.y);
-      const C Q = mkc<C>(rr1.x - c1 * qn.x, rr1.y - c1 * qn.y);
-      qn = Q;
-      qx[0] = P.x;
-      qx[1] = P.y;
-      qi[2] = Q.x;
-      qi[3] = Q.y;
+#pragma unroll
+    for (int i = kW - 2; i >= 0; --i) {
+      const C P = mkc<C>(r0v[i].x - c0[i] * qn.x, r0v[i].y - c0[i] * qn.y);
+      qn = mkc<C>(r1v[i].x - c1[i] * qn.x, r1v[i].y - c1[i] * qn.y);
+      if (w == i + 1) Xl = P;
+      if (w == i) Xr = qn;
     }
-    rw[0] = S(0);
-    rw[1] = S(0);
-    rw[(kCnSeg - 1) * 8 + 2] = S(0);
-    rw[(kCnSeg - 1) * 8 + 3] = S(0);
   }
-  wave_lds_sync();
-  const C XL = mkc<C>(rw[p * 8 + 0], rw[p * 8 + 1]);
-  const C XR = mkc<C>(rw[p * 8 + 2], rw[p * 8 + 3]);
+  // X_L = L_{p-1}, X_R = F_{p+1}, at the wave's ends X_l and X_r
+  yf = mkc<C>(yf.x - vf * Xl.x - wf * Xr.x, yf.y - vf * Xl.y - wf * Xr.y);
+  yl = mkc<C>(yl.x - vl * Xl.x - wl * Xr.x, yl.y - vl * Xl.y - wl * Xr.y);
+  C XL = mkc<C>(__shfl_up(yl.x, kCnSys), __shfl_up(yl.y, kCnSys));
+  C XR = mkc<C>(__shfl_down(yf.x, kCnSys), __shfl_down(yf.y, kCnSys));
+  XL = mkc<C>(p > 0 ? XL.x : Xl.x, p > 0 ? XL.y : Xl.y);
+  XR = mkc<C>(p < kCnSeg - 1 ? XR.x : Xr.x, p < kCnSeg - 1 ? XR.y : Xr.y);
+  asm volatile("" ::: "memory");
   // the segment's system with the boundary terms on the right: forward-swept
   // d''_r = d'_r - X_L v'_r - X_R w'_r (w'_r = 0 below the last row, cp_{R-1}
   // there), then the backward sweep x_r = d''_r - cp_r x_{r+1}
@@ -235,14 +278,20 @@ __global__ void __launch_bounds__(kCnThreads) k_cn_solve(const double *__restric
                                                        const double *__restrict__ alpha, const C *__restrict__ rhs,
                                                        C *__restrict__ x, int ny, long long nsys) {
   using S = Sc<C>;
-  __shared__ S red[(kCnThreads / 64) * 64 * 8];
-  __shared__ S tab[2 * kCnMaxNy];
-  for (int j = threadIdx.x; j < ny; j += blockDim.x) {
-    tab[j] = S(sl[j]);
-    tab[ny + j] = S(su[j]);
+  // rows of the three coefficients over alpha: sl without the coupling of row
+  // 0, su without that of row ny-1, and sl + su; zero rows (identity) from ny
+  // to the segments' end, so that no sweep tests its row
+  constexpr int kRows = SEG * kCnRows;
+  __shared__ S tab[3 * kRows];
+  __shared__ S xch[(kCnThreads / 64) * cn_systems(SEG) * 8];
+  for (int j = threadIdx.x; j < kRows; j += blockDim.x) {
+    const S l = j < ny ? S(sl[j]) : S(0), u = j < ny ? S(su[j]) : S(0);
+    tab[j] = j == 0 ? S(0) : l;
+    tab[kRows + j] = j == ny - 1 ? S(0) : u;
+    tab[2 * kRows + j] = l + u;
   }
   __syncthreads();
-  cn_solve_wave<kCnRows, SEG, C>(alpha, rhs, x, ny, nsys, red, tab, tab + ny);
+  cn_solve_block<kCnRows, SEG, C>(alpha, rhs, x, ny, nsys, tab, xch);
 }
 
 // ---------------------------------------------------------------------------
@@ -572,25 +621,24 @@ int dh_cn_solve_batched_dev(const double *sl, const double *su, const double *al
   if (nsys <= 0) return fail(DH_EARG, "nsys must be positive");
   if ((nsys + 7) / 8 > 0x7fffffffLL || (long long)ny * nsys > (1LL << 40)) return fail(DH_EARG, "too many systems");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // 16 lanes of 9 rows per system (ny <= 144) or 32 (ny <= 288)
-  const dim3 b(kCnThreads);
-  if (ny <= 16 * kCnRows) {
-    const dim3 g((unsigned)((nsys + 15) / 16));  // 4 waves of 4 systems
+  auto launch = [&](auto seg) {
+    constexpr int SEG = decltype(seg)::value, per = cn_systems(SEG);
+    const dim3 g((unsigned)((nsys + per - 1) / per)), b(kCnThreads);
     if (fp32)
-      hipLaunchKernelGGL((k_cn_solve<16, float2>), g, b, 0, st, sl, su, alpha, (const float2 *)rhs, (float2 *)x,
+      hipLaunchKernelGGL((k_cn_solve<SEG, float2>), g, b, 0, st, sl, su, alpha, (const float2 *)rhs, (float2 *)x,
                          (int)ny, (long long)nsys);
     else
-      hipLaunchKernelGGL((k_cn_solve<16, double2>), g, b, 0, st, sl, su, alpha, (const double2 *)rhs, (double2 *)x,
+      hipLaunchKernelGGL((k_cn_solve<SEG, double2>), g, b, 0, st, sl, su, alpha, (const double2 *)rhs, (double2 *)x,
                          (int)ny, (long long)nsys);
-  } else {
-    const dim3 g((unsigned)((nsys + 7) / 8));  // 4 waves of 2 systems
-    if (fp32)
-      hipLaunchKernelGGL((k_cn_solve<32, float2>), g, b, 0, st, sl, su, alpha, (const float2 *)rhs, (float2 *)x,
-                         (int)ny, (long long)nsys);
-    else
-      hipLaunchKernelGGL((k_cn_solve<32, double2>), g, b, 0, st, sl, su, alpha, (const double2 *)rhs, (double2 *)x,
-                         (int)ny, (long long)nsys);
-  }
+  };
+  if (ny <= 4 * kCnRows)
+    launch(std::integral_constant<int, 4>{});
+  else if (ny <= 8 * kCnRows)
+    launch(std::integral_constant<int, 8>{});
+  else if (ny <= 16 * kCnRows)
+    launch(std::integral_constant<int, 16>{});
+  else
+    launch(std::integral_constant<int, 32>{});
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(DH_EHIP, hipGetErrorString(e));
   return DH_OK;
