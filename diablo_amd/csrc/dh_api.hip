@@ -344,11 +344,6 @@ int dh_create(const dh_params *p, dh_ctx **out) {
   ACHK(dalloc(&c.fac.tb, 3 * (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.tc, 3 * (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.tr, 3 * (size_t)c.nfields * nyy));
-  {
-    const int rows = g.ny - 1;  // Poisson rows 2..NY swept per mode
-    const int sl = (rows + kRdsSeg - 1) / kRdsSeg;
-    c.rd_seg = (sl <= kRdsRows) ? sl : 0;
-  }
   c.fac.nseg = (nyy <= 4 * (size_t)kSegRows) ? 4 : 8;
   c.fac.seg_rows = (int)((nyy + c.fac.nseg - 1) / c.fac.nseg);
   ACHK(dalloc(&c.fac.isbc, (size_t)c.nfields * nyy));

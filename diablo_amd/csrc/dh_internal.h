@@ -75,8 +75,11 @@ struct Clock {
 // is split into 4 (NY+2 <= 144) or 8 such segments.
 constexpr int kSegRows = 36;
 constexpr int kStepsPerGraph = 8;  // time steps captured in one graph for long runs
-// Segments of one (kx,kz) mode's pressure-Poisson sweep over rows 2..NY, one
-// lane each, and the most rows a segment holds in registers.
+// Most rows 2..NY of one (kx,kz) mode's pressure-Poisson sweep that a thread
+// of REM_DIV holds in registers (23 of them per row).
+constexpr int kRdRows = 5;
+// The mixed form's REM_DIV: segments of a mode's sweep, one lane each, and
+// the most rows a segment holds in registers.
 constexpr int kRdsSeg = 8;
 constexpr int kRdsRows = 17;
 // Output k = t + 8 k2 of a register row transform (NX = 128) is stored only
@@ -165,7 +168,6 @@ struct Ctx {
   double *rd_ta = nullptr;      // REM_DIV sweep multipliers [NY+2][pf]
   double *rd_tb = nullptr;      // REM_DIV sweep pivots      [NY+2][pf]
   double *rd_tr = nullptr;      // REM_DIV 1/pivots          [NY+2][pf]
-  int rd_seg = 0;               // rows per REM_DIV sweep segment (0: one sequential sweep per mode)
   double *stats = nullptr;      // dh_save_stats profiles [DH_NSTATS][NY+2]
   Clock *clock = nullptr;
   RealFactors fac{};

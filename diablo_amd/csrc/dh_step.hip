@@ -1200,7 +1200,8 @@ struct RemDivArgs {
   double2 *phi;
   const double *rl, *ru;  // 1/(DY(J)DYF(J)), 1/(DY(J+1)DYF(J))
   double *ta, *tb, *tr;   // sweep multipliers, pivots, 1/pivots [J][mode]
-  int seg;                // rows per sweep segment; 0: one sequential sweep
+  int seg;                // rows per thread, at most kRdRows
+  int seg_mixed;          // mixed form: rows per sweep segment; 0: one sequential sweep
   // the step boundary after a step's last substep (diablo.f:66-110): TIME
   // += DELTA_T (bnd_end), TIME_STEP += 1 (bnd_begin), by one thread; no
   // thread of the launch reads TIME or TIME_STEP
@@ -1245,6 +1246,264 @@ __global__ void __launch_bounds__(256) k_rem_div_factors(RemDivArgs a) {
   }
 }
 
+// One pressure-Poisson solve per (kx,kz) mode: divergence (channel.f:1137-
+// 1143), the sweeps of THOMAS_FORWARD/BACKWARD_COMPLEX_MPI on the tabulated
+// multipliers and pivots (mpi.f:736-747, 838-856), projection and CP update
+// (channel.f:1185-1210, 1059-1065).  A block takes kRdtModes modes (128 B of
+// a Fourier row), G threads per mode, thread rg the rows [2 + rg seg, 1 + (rg
+// + 1) seg] (capped at NY) with everything they need in registers: velocity,
+// pressure and tables, read once.  Both recurrences are affine in the value
+// they carry in, G_J = V_J + A_J G_{J-1} and X_J = (G_J - U_J X_{J+1}) / B_J:
+// each thread forms its rows' map from a zero carry, the maps are composed
+// by a scan over the wave's 8 row groups and over the block's waves, and the
+// thread repeats its rows from the carry that gives, in the reference's
+// operations.  X = 0 where B = 0 (the sweep's guard), U_NY = 0, and row 1 is
+// set from row 2.
+//
+// What bounds it: memory where the modes fill the chip (71 MB in 16.5 us at
+// 128 x 129 x 128, 0.50 GB in 141 us at 256 x 193 x 256), the chain of loads,
+// two scans and stores where they do not (13.4 us at 256 x 257 x 4, 9.2 at
+// 64 x 97 x 64).  With eight lanes sweeping 17 rows each (NY <= 137) or one
+// lane all rows beyond, operands in LDS and the other waves idle, the same
+// launches took 22, 220, 48 and 15.3 us.
+constexpr int kRdtModes = 8;
+
+template <int G>
+struct RdShared {
+  double wa[2][G / 8][kRdtModes];      // a wave's map: factor and
+  double2 wb[2][G / 8][kRdtModes];     // constant, forward and backward
+  double2 last[G][kRdtModes];          // phi in a thread's last row
+};
+
+// nb blocks of modes, this one lin
+template <int G>
+__device__ __forceinline__ void rem_div_thomas_body(const RemDivArgs &a, int nb, int lin, RdShared<G> &sh) {
+#pragma clang fp contract(off)
+  constexpr int R = kRdRows, NW = G / 8;
+  if (lin == 0 && threadIdx.x == 0) {
+    if (a.bnd_end) a.clk->time = a.clk->time + a.clk->dt;
+    if (a.bnd_begin) a.clk->time_step += 1;
+  }
+  const Geo &g = a.g;
+  const int NY = g.ny, seg = a.seg;
+  const int lane = threadIdx.x % kRdtModes, rg = threadIdx.x / kRdtModes, rw = rg & 7, w = rg >> 3;
+  // mode groups dealt so that XCD x (blocks x, x+8, ...) takes a contiguous
+  // range: neighbouring groups share the cache lines their rows straddle
+  int grp;
+  {
+    const int x = lin & 7, q = nb >> 3, r = nb & 7;
+    grp = x * q + min(x, r) + (lin >> 3);
+  }
+  const int m = grp * kRdtModes + lane;
+  const bool live = m < g.pf;
+  const long long pf = g.pf;
+  int kx = 0, kzp = 0;
+  if (live) {
+    kzp = (int)fdiv((unsigned)m, g.f_nkx1);
+    kx = m - kzp * g.nkx1;
+  }
+  const double kxv = g.kx[kx], kzv = g.kz[kzp];
+  const bool mean = (kx == 0 && kzp == 0);
+  const bool upd = a.rk >= 0;
+  const int r0 = 2 + rg * seg, r1 = min(NY, r0 + seg - 1);
+  const double2 zero = make_double2(0.0, 0.0);
+  // rows q of this thread: J = r0 + q <= r1
+  auto has = [&](int q) { return live && r0 + q <= r1; };
+  double2 u1[R], u2[R], u3[R], pc[R], u2e = zero, g1 = zero, g3 = zero;
+  double ta[R], tb[R], tr[R], U[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    u1[q] = u2[q] = u3[q] = pc[q] = zero;
+    ta[q] = 1.0;
+    tb[q] = tr[q] = 1.0;
+    U[q] = 0.0;
+    if (has(q)) {
+      const int J = r0 + q;
+      const long long o = pf * J + m;
+      u1[q] = a.cin[0][o];
+      u2[q] = a.cin[1][o];
+      u3[q] = a.cin[2][o];
+      if (upd) pc[q] = a.cp[o];
+      ta[q] = a.ta[o];
+      tb[q] = a.tb[o];
+      tr[q] = a.tr[o];
+      if (J < NY) U[q] = a.ru[J];
+    }
+  }
+  if (live && r0 <= r1 && r1 < NY) u2e = a.cin[1][pf * (r1 + 1) + m];
+  if (live && rg == 0) {  // row 1 is group 0's too
+    g1 = a.cin[0][pf + m];
+    g3 = a.cin[2][pf + m];
+  }
+  // right-hand sides V of rows 2..NY-1 (row NY is a BC row with zero
+  // right-hand side) and the group's forward map G_out = ha G_in + hb
+  double2 v[R];
+  double fa = 1.0;
+  double2 fb = zero;
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    v[q] = zero;
+    if (has(q)) {
+      const int J = r0 + q;
+      if (J < NY) {
+        double2 up = u2e;
+        if (q + 1 < R && J < r1) up = u2[q + 1 < R ? q + 1 : q];
+        const double2 t1 = cmul_ik(kxv, u1[q]), t3 = cmul_ik(kzv, u3[q]);
+        const double d = g.dyf[J], rd = g.rdyf[J];
+        v[q] = make_double2(t1.x + div_by_recip(up.x - u2[q].x, d, rd) + t3.x,
+                            t1.y + div_by_recip(up.y - u2[q].y, d, rd) + t3.y);
+      }
+      fb = make_double2(v[q].x + ta[q] * fb.x, v[q].y + ta[q] * fb.y);
+      fa = ta[q] * fa;
+    }
+  }
+  // inclusive composition over the wave's groups (UP: from group 0 on, else
+  // from the last group down), the waves' maps through LDS, and the value
+  // carried into this group
+  auto carry = [&](auto up_, double ca, double2 cb, int k) {
+    constexpr bool UP = decltype(up_)::value;
+#pragma unroll
+    for (int s = 1; s < 8; s *= 2) {
+      const int d = kRdtModes * s;
+      const double pa = UP ? __shfl_up(ca, d) : __shfl_down(ca, d);
+      const double px = UP ? __shfl_up(cb.x, d) : __shfl_down(cb.x, d);
+      const double py = UP ? __shfl_up(cb.y, d) : __shfl_down(cb.y, d);
+      if (UP ? rw >= s : rw + s < 8) {
+        cb = make_double2(ca * px + cb.x, ca * py + cb.y);
+        ca = ca * pa;
+      }
+    }
+    if (rw == (UP ? 7 : 0)) {
+      sh.wa[k][w][lane] = ca;
+      sh.wb[k][w][lane] = cb;
+    }
+    lds_barrier();
+    double2 X = zero;
+#pragma unroll
+    for (int i = 0; i < NW - 1; ++i) {
+      const int j = UP ? i : NW - 1 - i;
+      if (UP ? j < w : j > w) {
+        const double wa = sh.wa[k][j][lane];
+        const double2 wb = sh.wb[k][j][lane];
+        X = make_double2(wa * X.x + wb.x, wa * X.y + wb.y);
+      }
+    }
+    const double pa = UP ? __shfl_up(ca, kRdtModes) : __shfl_down(ca, kRdtModes);
+    const double px = UP ? __shfl_up(cb.x, kRdtModes) : __shfl_down(cb.x, kRdtModes);
+    const double py = UP ? __shfl_up(cb.y, kRdtModes) : __shfl_down(cb.y, kRdtModes);
+    if (rw != (UP ? 0 : 7)) X = make_double2(pa * X.x + px, pa * X.y + py);
+    return X;
+  };
+  double2 c = carry(std::true_type{}, fa, fb, 0);  // G_{r0-1} (G_1 = 0)
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    if (has(q)) {
+      c = make_double2(v[q].x + ta[q] * c.x, v[q].y + ta[q] * c.y);
+      v[q] = c;
+    }
+  }
+  // the group's backward map X_{r0} = ba X_{r1+1} + bb
+  auto back = [&](int q, double2 x) {
+    const double xr = div_by_recip(v[q].x - U[q] * x.x, tb[q], tr[q]);
+    const double xi = div_by_recip(v[q].y - U[q] * x.y, tb[q], tr[q]);
+    return make_double2((tb[q] != 0.0) ? xr : 0.0, (tb[q] != 0.0) ? xi : 0.0);
+  };
+  double ba = 1.0;
+  double2 bb = zero;
+#pragma unroll
+  for (int q = R - 1; q >= 0; --q) {
+    if (has(q)) {
+      bb = back(q, bb);
+      ba = (tb[q] != 0.0) ? div_by_recip(-U[q], tb[q], tr[q]) * ba : 0.0;
+    }
+  }
+  c = carry(std::false_type{}, ba, bb, 1);  // X_{r1+1} (nothing above row NY)
+  double2 top = zero;
+#pragma unroll
+  for (int q = R - 1; q >= 0; --q) {
+    if (has(q)) {
+      c = back(q, c);
+      v[q] = c;
+      if (r0 + q == r1) top = c;
+    }
+  }
+  sh.last[rg][lane] = top;
+  lds_barrier();
+  if (!live) return;
+  // phi below the group's first row; row 1: B=1, G=0, U = 0 (mean mode) or -1
+  const double U1 = mean ? 0.0 : -1.0;
+  const double2 phi1 = make_double2((0.0 - U1 * v[0].x) / 1.0, (0.0 - U1 * v[0].y) / 1.0);
+  double2 pm = rg == 0 ? phi1 : sh.last[rg > 0 ? rg - 1 : 0][lane];
+  const double hb = upd ? (a.cp_old ? a.clk->h_cp : a.clk->h_bar[a.rk]) : 1.0;
+  const double rhb = 1.0 / hb;
+  auto project13 = [&](int J, double2 c1, double2 c3, double2 phi) {
+    const long long o = pf * J + m;
+    if (!upd) a.phi[o] = phi;  // REM_DIV alone leaves phi (CR1) behind
+    double2 t = cmul_ik(kxv, phi);
+    a.cu[0][o] = make_double2(c1.x - t.x, c1.y - t.y);
+    t = cmul_ik(kzv, phi);
+    a.cu[2][o] = make_double2(c3.x - t.x, c3.y - t.y);
+  };
+  if (rg == 0) project13(1, g1, g3, phi1);
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    if (has(q)) {
+      const int J = r0 + q;
+      const long long o = pf * J + m;
+      const double2 phi = v[q];
+      project13(J, u1[q], u3[q], phi);
+      const double d = g.dy[J], rd = g.rdy[J];
+      a.cu[1][o] = make_double2(u2[q].x - div_by_recip(phi.x - pm.x, d, rd), u2[q].y - div_by_recip(phi.y - pm.y, d, rd));
+      if (upd)
+        a.cp[o] = make_double2(pc[q].x + div_by_recip(phi.x, hb, rhb), pc[q].y + div_by_recip(phi.y, hb, rhb));
+      pm = phi;
+    }
+  }
+  // planes the projection leaves alone (the ghost planes 0 and NY+1, and
+  // plane 1 of CU2) pass from the transformed velocity unchanged
+  if (a.cin[0] != a.cu[0]) {
+    auto pass = [&](int f, int J) { a.cu[f][pf * J + m] = a.cin[f][pf * J + m]; };
+    if (rg == 0) {
+      pass(0, 0);
+      pass(1, 0);
+      pass(2, 0);
+      pass(1, 1);
+    } else if (rg == G - 1) {
+      pass(0, NY + 1);
+      pass(1, NY + 1);
+      pass(2, NY + 1);
+    }
+  }
+}
+template <int G>
+__global__ void __launch_bounds__(kRdtModes * G) k_rem_div_thomas(RemDivArgs a) {
+  __shared__ RdShared<G> sh;
+  rem_div_thomas_body<G>(a, gridDim.x, blockIdx.x, sh);
+}
+template <int G>
+__global__ void __launch_bounds__(kRdtModes * G) k_rem_div_thomas_b(const RemDivArgs *__restrict__ av) {
+  __shared__ RdShared<G> sh;
+  rem_div_thomas_body<G>(av[blockIdx.z], gridDim.x, blockIdx.x, sh);
+}
+// REM_DIV with the CN tables of a new DELTA_T in the grid's last ncn blocks
+// (the substep after COURANT: the tables serve the next substep's solve,
+// and REM_DIV reads none of what they write).
+template <int G>
+__global__ void __launch_bounds__(kRdtModes * G) k_rem_div_thomas_cn(RemDivArgs a, CnArgs cn, int ncn) {
+  __shared__ RdShared<G> sh;
+  const int nrd = (int)gridDim.x - ncn;
+  if ((int)blockIdx.x >= nrd) {
+    cn_tables_body(cn.clk, cn.in, cn.fac, (int)blockIdx.x - nrd);
+    return;
+  }
+  rem_div_thomas_body<G>(a, nrd, blockIdx.x, sh);
+}
+
+// REM_DIV of the mixed form: the same solve with its rows' rounding as it was
+// before the sweeps were split over G threads per mode.  The FP32 transforms
+// carry a last-bit difference of CU to 1e-7 of every field within two steps
+// (each flipped rounding flips others), so a faster FP64 sweep would change
+// that form's results by as much as FP32 does; it keeps these kernels.
 // One pressure-Poisson solve per (kx,kz) mode.  All threads stage the
 // divergence (channel.f:1137-1143) and the mode's multipliers and pivots of
 // kRdtModes modes into LDS; one lane per mode runs the forward and backward
@@ -1252,7 +1511,6 @@ __global__ void __launch_bounds__(256) k_rem_div_factors(RemDivArgs a) {
 // (channel.f:1185-1210, 1059-1065).  The sweeps read their operands
 // kRdtAhead rows ahead without bounds tests (kRdtPad rows of padding below
 // and above rows 0..NY), so nothing in the recurrence waits on LDS.
-constexpr int kRdtModes = 8;
 
 // The sweeps of one mode split into kRdsSeg segments of `seg` rows
 // [2 + s seg, 1 + (s+1) seg] (capped at NY), segment s on lane s*kRdtModes
@@ -1361,7 +1619,7 @@ constexpr int kRdtPad = 16;  // >= 4 * kRdtAhead - 1: the sweeps read up to 4 kR
 constexpr int kRdtRegRows = 5;
 
 // nb blocks of modes, this one lin
-__device__ __forceinline__ void rem_div_thomas_body(const RemDivArgs &a, int nb, int lin) {
+__device__ __forceinline__ void rem_div_mixed_body(const RemDivArgs &a, int nb, int lin) {
 #pragma clang fp contract(off)
   extern __shared__ double st[];
   if (lin == 0 && threadIdx.x == 0) {
@@ -1457,8 +1715,8 @@ __device__ __forceinline__ void rem_div_thomas_body(const RemDivArgs &a, int nb,
     stage_row(J, c1, c2, c3, c2p, ta, tb, tr);
   }
   lds_barrier();
-  if (a.seg > 0) {
-    if (rg < kRdsSeg) rem_div_sweep_seg(a.seg, rg, lane, NY, mean, Gs, As, Bs, Rs, ru);
+  if (a.seg_mixed > 0) {
+    if (rg < kRdsSeg) rem_div_sweep_seg(a.seg_mixed, rg, lane, NY, mean, Gs, As, Bs, Rs, ru);
   } else if (rg == 0) {
     // forward: G_J = V_J + A_J G_{J-1}, J = 2..NY, G_1 = 0.  Two register
     // sets of kRdtAhead rows alternate: one set's rows are computed while
@@ -1592,20 +1850,20 @@ __device__ __forceinline__ void rem_div_thomas_body(const RemDivArgs &a, int nb,
 // Two blocks per CU (the velocity rows held across the sweep take the
 // registers of a third): 512 resident blocks cover the 457 of a 128 x 128
 // plane's modes at once.
-__global__ void __launch_bounds__(256) k_rem_div_thomas(RemDivArgs a) { rem_div_thomas_body(a, gridDim.x, blockIdx.x); }
-__global__ void __launch_bounds__(256) k_rem_div_thomas_b(const RemDivArgs *__restrict__ av) {
-  rem_div_thomas_body(av[blockIdx.z], gridDim.x, blockIdx.x);
+__global__ void __launch_bounds__(256) k_rem_div_mixed(RemDivArgs a) { rem_div_mixed_body(a, gridDim.x, blockIdx.x); }
+__global__ void __launch_bounds__(256) k_rem_div_mixed_b(const RemDivArgs *__restrict__ av) {
+  rem_div_mixed_body(av[blockIdx.z], gridDim.x, blockIdx.x);
 }
 // REM_DIV with the CN tables of a new DELTA_T in the grid's last ncn blocks
 // (the substep after COURANT: the tables serve the next substep's solve,
 // and REM_DIV reads none of what they write).
-__global__ void __launch_bounds__(256) k_rem_div_thomas_cn(RemDivArgs a, CnArgs cn, int ncn) {
+__global__ void __launch_bounds__(256) k_rem_div_mixed_cn(RemDivArgs a, CnArgs cn, int ncn) {
   const int nrd = (int)gridDim.x - ncn;
   if ((int)blockIdx.x >= nrd) {
     cn_tables_body(cn.clk, cn.in, cn.fac, (int)blockIdx.x - nrd);
     return;
   }
-  rem_div_thomas_body(a, nrd, blockIdx.x);
+  rem_div_mixed_body(a, nrd, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -2295,10 +2553,14 @@ hipError_t launch_solve_les_range(Ctx &c, int rk, int courant, int f0, int f1, h
   return klaunch(c, (const void *)k_solve_les, nullptr, grid, dim3(kLesSolveThreads), 0, st, a);
 }
 
-static size_t rem_div_thomas_lds(const Ctx &c) {
+static size_t rem_div_mixed_lds(const Ctx &c) {
   const size_t ntot = c.g.ny + 1 + 2 * kRdtPad;
   return ntot * kRdtModes * 5 * sizeof(double) + ntot * sizeof(double);
 }
+
+// Threads per mode of REM_DIV: 32, or 64 beyond the rows that 32 hold.
+static int rem_div_groups(const Ctx &c) { return c.g.ny - 1 <= 32 * kRdRows ? 32 : 64; }
+static_assert(8 * kSegRows - 3 <= 64 * kRdRows, "every NY of dh_create fits 64 row groups");
 
 static RemDivArgs make_rem_div_args(Ctx &c, int rk) {
   RemDivArgs a{};
@@ -2317,7 +2579,10 @@ static RemDivArgs make_rem_div_args(Ctx &c, int rk) {
   a.ta = c.rd_ta;
   a.tb = c.rd_tb;
   a.tr = c.rd_tr;
-  a.seg = c.rd_seg;
+  const int ng = rem_div_groups(c);
+  a.seg = (c.g.ny - 1 + ng - 1) / ng;
+  const int sl = (c.g.ny - 1 + kRdsSeg - 1) / kRdsSeg;
+  a.seg_mixed = (sl <= kRdsRows) ? sl : 0;
   return a;
 }
 
@@ -2332,8 +2597,14 @@ hipError_t launch_rem_div(Ctx &c, int rk, int bnd_end, int bnd_begin) {
   a.bnd_end = bnd_end;
   a.bnd_begin = bnd_begin;
   const int nb = (c.g.pf + kRdtModes - 1) / kRdtModes;
-  return klaunch(c, (const void *)k_rem_div_thomas, (const void *)k_rem_div_thomas_b, dim3(nb), dim3(256),
-                 (unsigned)rem_div_thomas_lds(c), c.stream, a);
+  if (c.mixed && rk >= 0)
+    return klaunch(c, (const void *)k_rem_div_mixed, (const void *)k_rem_div_mixed_b, dim3(nb), dim3(256),
+                   (unsigned)rem_div_mixed_lds(c), c.stream, a);
+  if (rem_div_groups(c) == 32)
+    return klaunch(c, (const void *)k_rem_div_thomas<32>, (const void *)k_rem_div_thomas_b<32>, dim3(nb),
+                   dim3(kRdtModes * 32), 0, c.stream, a);
+  return klaunch(c, (const void *)k_rem_div_thomas<64>, (const void *)k_rem_div_thomas_b<64>, dim3(nb),
+                 dim3(kRdtModes * 64), 0, c.stream, a);
 }
 
 // REM_DIV and the CN tables for the DELTA_T COURANT just set, in one launch
@@ -2345,9 +2616,14 @@ static hipError_t launch_rem_div_cn(Ctx &c, int rk, int bnd_end, int bnd_begin) 
   a.bnd_begin = bnd_begin;
   const CnArgs cn{c.clock, make_factor_in(c), c.fac};
   const int nb = (c.g.pf + kRdtModes - 1) / kRdtModes, ncn = 3 * c.nfields;
-  const size_t lrd = rem_div_thomas_lds(c), lcn = (size_t)8 * (c.g.ny + 2) * sizeof(double);
-  const size_t lds = lrd > lcn ? lrd : lcn;
-  hipLaunchKernelGGL(k_rem_div_thomas_cn, dim3(nb + ncn), dim3(256), (unsigned)lds, c.stream, a, cn, ncn);
+  const unsigned lds = (unsigned)(8 * (c.g.ny + 2) * sizeof(double));  // the tables' blocks
+  if (c.mixed) {
+    const unsigned lrd = (unsigned)rem_div_mixed_lds(c);
+    hipLaunchKernelGGL(k_rem_div_mixed_cn, dim3(nb + ncn), dim3(256), lrd > lds ? lrd : lds, c.stream, a, cn, ncn);
+  } else if (rem_div_groups(c) == 32)
+    hipLaunchKernelGGL(k_rem_div_thomas_cn<32>, dim3(nb + ncn), dim3(kRdtModes * 32), lds, c.stream, a, cn, ncn);
+  else
+    hipLaunchKernelGGL(k_rem_div_thomas_cn<64>, dim3(nb + ncn), dim3(kRdtModes * 64), lds, c.stream, a, cn, ncn);
   return hipGetLastError();
 }
 
@@ -2477,7 +2753,7 @@ hipError_t launch_step_boundary(Ctx &c, bool end_prev, bool begin_next) {
 }
 
 hipError_t prepare_step_kernels(Ctx &c) {
-  if ((c.lds_bytes > kLdsMax && !c.gp) || (long long)rem_div_thomas_lds(c) > kLdsMax) return hipErrorInvalidValue;
+  if ((c.lds_bytes > kLdsMax && !c.gp) || (long long)rem_div_mixed_lds(c) > kLdsMax) return hipErrorInvalidValue;
   const void *fns[] = {(const void *)k_nonlinear<true, kNlRegQ>,    (const void *)k_nonlinear<false, kMaxQ>,
                        (const void *)k_nonlinear<true, kNlRegQ, true>, (const void *)k_nonlinear<false, kMaxQ, true>,
                        (const void *)k_nonlinear<false, kMaxQ, false, 512>,
@@ -2486,8 +2762,8 @@ hipError_t prepare_step_kernels(Ctx &c) {
                        (const void *)k_nonlinear32<true, kNlRegQ>,  (const void *)k_nonlinear32<false, kMaxQ>,
                        (const void *)k_nonlinear_b<true, kNlRegQ>,  (const void *)k_nonlinear_b<false, kMaxQ>,
                        (const void *)k_nonlinear32_b<true, kNlRegQ>, (const void *)k_nonlinear32_b<false, kMaxQ>,
-                       (const void *)k_rem_div_thomas,              (const void *)k_rem_div_thomas_b,
-                       (const void *)k_rem_div_thomas_cn};
+                       (const void *)k_rem_div_mixed,               (const void *)k_rem_div_mixed_b,
+                       (const void *)k_rem_div_mixed_cn};
   for (const void *fn : fns) {
     const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
     if (e != hipSuccess) return e;
