@@ -597,6 +597,303 @@ __device__ __forceinline__ void nonlinear_pass(const StepArgs &a, C *A) {
     plane_store_phys(A, g, T, dst);
   }
 }
+
+// What the RK combination of component c at plane J (channel.f:88-167,
+// 581-595; scalars 254-270, 723-729) and the explicit half of its y-viscous
+// term in Fourier space (channel.f:606-626, 739-747; as in nonlinear_pass)
+// take besides the mode's coefficients.
+struct RkRow {
+  double T3, T4, T5, coefv;
+  double ey0, ey1, ey2, rey0, rey1, rey2;  // weights of C(J+1)-C(J), C(J)-C(J-1) and the outer divisor
+  double dy, rdy;
+};
+__device__ __forceinline__ RkRow rk_row(const StepArgs &a, int c, int J) {
+  const Geo &g = a.g;
+  RkRow r;
+  const double hb = a.clk->h_bar[a.rk];
+  r.T3 = a.clk->zeta_bar[a.rk] * hb;
+  r.T4 = hb;
+  r.T5 = a.clk->beta_bar[a.rk] * hb;
+  r.coefv = (c < 3) ? (a.nu * hb / 2.0) * a.nu_v_scale : ((a.nu * hb / 2.0) / a.pr[c - 3]) * a.nu_v_scale;
+  const bool v = c == 1;
+  r.ey0 = v ? g.dyf[J] : g.dy[J + 1];
+  r.ey1 = v ? g.dyf[J - 1] : g.dy[J];
+  r.ey2 = v ? g.dy[J] : g.dyf[J];
+  r.rey0 = v ? g.rdyf[J] : g.rdy[J + 1];
+  r.rey1 = v ? g.rdyf[J - 1] : g.rdy[J];
+  r.rey2 = v ? g.rdy[J] : g.rdyf[J];
+  r.dy = g.dy[J];
+  r.rdy = g.rdy[J];
+  return r;
+}
+// One mode's coefficients that the combination reads at plane J (and its
+// neighbours): C(J), C(J-1), C(J+1), the old CF, CP(J), CP(J-1).
+struct RkMode {
+  double2 c0, cm1, cp1, old, p0, pm;
+};
+__device__ __forceinline__ RkMode rk_load(const StepArgs &a, int c, long long o) {
+  const long long pf = a.g.pf;
+  const double2 zero = make_double2(0.0, 0.0);
+  const double2 *CF = (c < 3) ? a.cf[c] : a.cfth + (c - 3) * a.cfs;
+  const double2 *CC = (c < 3) ? a.cu[c] : a.cth + (c - 3) * a.cfs;
+  RkMode m;
+  m.c0 = CC[o];
+  m.cm1 = CC[o - pf];
+  m.cp1 = CC[o + pf];
+  m.old = (a.rk > 0) ? CF[o] : zero;
+  m.p0 = (c < 3) ? a.cp[o] : zero;
+  m.pm = (c == 1) ? a.cp[o - pf] : zero;
+  return m;
+}
+// CR of the mode without its new CF (which joins as T5 CF); kk: KX (U1) or KZ
+// (U3) of the pressure gradient, mean: the (0,0) mode (SGS: LES, whose column
+// solve takes the explicit y-viscous half).
+template <bool SGS>
+__device__ __forceinline__ double2 rk_combine(const StepArgs &a, const RkRow &r, int c, double kk, bool mean,
+                                              const RkMode &m) {
+  double2 cr = m.c0;
+  if (a.rk > 0) cr = make_double2(cr.x + r.T3 * m.old.x, cr.y + r.T3 * m.old.y);
+  if (c == 0 || c == 2) {
+    const double2 ikp = cmul_ik(kk, m.p0);
+    cr = make_double2(cr.x - r.T4 * ikp.x, cr.y - r.T4 * ikp.y);
+    if (c == 0 && mean) {
+      if (a.f_type == 1)
+        cr.x = cr.x - r.T4 * a.px0;
+      else if (a.f_type == 2)
+        cr.x = cr.x - r.T4 * (a.px0 + a.amp_omega0 * cos(a.omega0 * a.clk->time));
+    }
+  } else if (c == 1) {
+    const double2 cs = make_double2(div_by_recip(m.p0.x - m.pm.x, r.dy, r.rdy), div_by_recip(m.p0.y - m.pm.y, r.dy, r.rdy));
+    cr = make_double2(cr.x - r.T4 * cs.x, cr.y - r.T4 * cs.y);
+  }
+  if constexpr (!SGS) {
+    const double2 ev = make_double2(
+        r.coefv * div_by_recip(div_by_recip(m.cp1.x - m.c0.x, r.ey0, r.rey0) - div_by_recip(m.c0.x - m.cm1.x, r.ey1, r.rey1), r.ey2, r.rey2),
+        r.coefv * div_by_recip(div_by_recip(m.cp1.y - m.c0.y, r.ey0, r.rey0) - div_by_recip(m.c0.y - m.cm1.y, r.ey1, r.rey1), r.ey2, r.rey2));
+    cr = make_double2(cr.x + ev.x, cr.y + ev.y);
+  }
+  return cr;
+}
+
+// The explicit Fourier terms of cf_init from coefficients loaded ahead: u the
+// component's own, x0 and x1 what it takes beside it (cf_load; the further
+// scalars of a velocity component are read here).
+__device__ __forceinline__ void cf_load(const StepArgs &a, int c, long long o, double2 &x0, double2 &x1) {
+  const double2 zero = make_double2(0.0, 0.0);
+  const bool th = a.n_th > 0;
+  if (c == 1) {
+    x0 = th ? a.cth[o] : zero;
+    x1 = th ? a.cth[o - a.g.pf] : zero;
+  } else if (c < 3) {
+    x0 = a.cu[2 - c][o];
+    x1 = th ? a.cth[o] : zero;
+  } else {
+    x0 = a.cu[0][o];
+    x1 = a.cu[2][o];
+  }
+}
+__device__ __forceinline__ double2 cf_terms(const StepArgs &a, int c, int J, double k2, bool mean, long long o,
+                                            double2 u, double2 x0, double2 x1) {
+  const Geo &g = a.g;
+  const double f = ((c < 3) ? a.nu : a.nu / a.pr[c - 3]) * kpow(k2, a.beta);
+  double2 cf = make_double2(-(f * u.x), -(f * u.y));
+  if (c >= 3) {
+    const double dx = a.drhodx[c - 3], dz = a.drhodz[c - 3];
+    return make_double2(cf.x - x0.x * dx - x1.x * dz, cf.y - x0.y * dx - x1.y * dz);
+  }
+  if (c != 1) {
+    const double ro = (c == 0) ? a.i_ro : -a.i_ro;
+    cf = make_double2(cf.x + ro * x0.x, cf.y + ro * x0.y);
+  }
+  for (int n = 0; n < a.n_th; ++n) {
+    const double2 *CTH = a.cth + n * a.cfs + o;
+    if (c == 1) {
+      if (mean) continue;  // plane mean skipped (channel.f:217-226)
+      const double2 t0 = n ? CTH[0] : x0, tm = n ? CTH[-g.pf] : x1;
+      const double s = a.ri[n] * a.grav_y;
+      const double d = 2.0 * g.dy[J], r = 0.5 * g.rdy[J];
+      cf = make_double2(cf.x + div_by_recip(s * (t0.x * g.dyf[J - 1] + tm.x * g.dyf[J]), d, r),
+                        cf.y + div_by_recip(s * (t0.y * g.dyf[J - 1] + tm.y * g.dyf[J]), d, r));
+    } else {
+      const double2 t = n ? CTH[0] : x1;
+      const double s = a.ri[n] * ((c == 0) ? a.grav_x : a.grav_z);
+      cf = make_double2(cf.x + s * t.x, cf.y + s * t.y);
+    }
+  }
+  return cf;
+}
+
+// The nonlinear pass for small planes (FP64): the terms of nonlinear_pass in
+// the same order, with the three products of a component side by side in
+// LDS (row z of product p at (3 z + p) LS), so that each pass of the
+// transforms runs once over all three instead of three times over one; the
+// inverse transform has a plane of its own behind them.  A plane of a few
+// hundred values gives a stage less than one butterfly per thread: the pass
+// is a chain of stages, barriers and loads, and what counts is its length.
+// Everything that the first of a thread's modes and samples need is requested
+// before the transform tables are staged, each sample once for all three
+// products; of the mode only CF's explicit terms and CR without the new CF
+// stay in registers through the transforms.
+//
+// What bounds it: that chain, and with four blocks of 256 threads on every CU
+// the issue of its LDS stages.  256 x 257 x 4 with a scalar: 46 us a launch
+// against 75 with the products one after another in blocks of 128 threads;
+// 64 x 65 x 4: 14.6 against 24.7.
+constexpr int kNlSmallThreads = 256;
+constexpr int kNlSmallSlots = 896;  // most complex values of a plane
+template <bool SGS>
+__device__ __forceinline__ void nonlinear_small(const StepArgs &a, double2 *A) {
+  const Geo &g = a.g;
+  // (plane, component) of this block as in nonlinear_pass
+  int J, c;
+  {
+    const int nblk = gridDim.x * gridDim.y, lin = blockIdx.x + blockIdx.y * gridDim.x;
+    const int x = lin & 7, q = nblk >> 3, r = nblk & 7;
+    const int w = x * q + min(x, r) + (lin >> 3);
+    const int jr = w / (int)gridDim.y;
+    J = __builtin_amdgcn_readfirstlane(a.j0 + jr);
+    c = __builtin_amdgcn_readfirstlane(a.c0 + w - jr * (int)gridDim.y);
+  }
+  int jlo = 2, jhi = g.ny;
+  if (c >= 3) {
+    jlo = a.jstart_th[c - 3];
+    jhi = a.jend_th[c - 3];
+  }
+  if (J < jlo || J > jhi) return;
+  const int nthr = blockDim.x, slots = g.nz * g.lw;
+  // a mode's coefficients and wavenumbers, and what remains of them once the
+  // terms that do not depend on the products are formed
+  struct Raw {
+    RkMode rk;
+    double2 x0, x1;
+    double kx, kz, k2;
+    int kzp, kxi;
+  };
+  struct Mode {
+    double2 cf, cr;
+    double kx, kz;
+    int kzp, kxi;
+  };
+  auto load_mode = [&](int m) {
+    Raw w;
+    w.kzp = (int)fdiv((unsigned)m, g.f_nkx1);
+    w.kxi = m - w.kzp * g.nkx1;
+    const long long o = (long long)J * g.pf + m;
+    w.rk = rk_load(a, c, o);
+    cf_load(a, c, o, w.x0, w.x1);
+    w.kx = g.kx[w.kxi];
+    w.kz = g.kz[w.kzp];
+    w.k2 = g.kx2[w.kxi] + g.kz2[w.kzp];
+    return w;
+  };
+  auto form_mode = [&](int m, const Raw &w) {
+    const RkRow rr = rk_row(a, c, J);
+    const long long o = (long long)J * g.pf + m;
+    const bool mean = w.kxi == 0 && w.kzp == 0;
+    Mode md{cf_terms(a, c, J, w.k2, mean, o, w.rk.c0, w.x0, w.x1),
+            rk_combine<SGS>(a, rr, c, (c == 0) ? w.kx : w.kz, mean, w.rk), w.kx, w.kz, w.kzp, w.kxi};
+    if constexpr (SGS) md.cf = cadd(md.cf, a.sgs[c * a.cfs + o]);
+    return md;
+  };
+  const int m0 = min((int)threadIdx.x, g.pf - 1);
+  const Raw w0 = load_mode(m0);
+  // the planes whose samples the three products take (make_prod's forms)
+  const double *up = static_cast<const double *>(a.uphys);
+  auto plane = [&](int f, int j) { return up + f * a.fs + (long long)j * g.pp; };
+  const double *pl[7];
+  if (c == 1) {  // U1, U3 at J, J-1; U2 at J+1, J, J-1
+    pl[0] = plane(0, J); pl[1] = plane(0, J - 1); pl[2] = plane(2, J); pl[3] = plane(2, J - 1);
+    pl[4] = plane(1, J + 1); pl[5] = plane(1, J); pl[6] = plane(1, J - 1);
+  } else {  // the component at J+1, J, J-1; U2 at J+1, J; the others at J
+    pl[0] = plane(c, J + 1); pl[1] = plane(c, J); pl[2] = plane(c, J - 1); pl[3] = plane(1, J + 1); pl[4] = plane(1, J);
+    pl[5] = plane(c < 3 ? 2 - c : 0, J);
+    pl[6] = plane(2, J);  // scalars: U3
+  }
+  const Prod<double2> p0 = make_prod<double2>(a, c, 0, J), p2 = make_prod<double2>(a, c, 2, J);
+  const int np = (c == 0 || c == 2) ? 6 : 7;
+  Tables T;
+  constexpr int B = 2;
+  for (int e0 = threadIdx.x; e0 < slots || e0 == (int)threadIdx.x; e0 += B * nthr) {
+    double2 v[B][7];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const long long off = 2 * (long long)min(e0 + b * nthr, slots - 1);
+#pragma unroll
+      for (int i = 0; i < 7; ++i)
+        if (i < np) v[b][i] = *reinterpret_cast<const double2 *>(pl[i] + off);
+    }
+    if (e0 == (int)threadIdx.x) T = load_tables_at(A + 4 * g.nz * g.ls, g);  // every thread once; ends on a barrier
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int e = e0 + b * nthr;
+      if (e < slots) {
+        const int z = (int)fdiv((unsigned)e, g.f_lw), xp = e - z * g.lw;
+        double2 *row = A + 3 * z * g.ls + T.posr[xp];
+        const double2 *s = v[b];
+        if (c == 1) {
+          row[0] = eval_raw<3, double2>(p0, ProdRaw<3, double2>{{s[0], s[1], s[5]}});
+          row[g.ls] = eval_raw<3, double2>(p0, ProdRaw<3, double2>{{s[2], s[3], s[5]}});
+          row[2 * g.ls] = eval_raw<4, double2>(p2, ProdRaw<4, double2>{{s[4], s[5], s[6]}});
+        } else {
+          row[0] = eval_raw<0, double2>(p0, ProdRaw<0, double2>{{s[5], s[1]}});
+          row[g.ls] = c < 3 ? eval_raw<1, double2>(p0, ProdRaw<1, double2>{{s[1]}})
+                            : eval_raw<0, double2>(p0, ProdRaw<0, double2>{{s[1], s[6]}});
+          row[2 * g.ls] = eval_raw<2, double2>(p2, ProdRaw<2, double2>{{s[0], s[1], s[2], s[3], s[4]}});
+        }
+      }
+    }
+  }
+  const Mode md0 = form_mode(m0, w0);
+  const double T5 = a.clk->beta_bar[a.rk] * a.clk->h_bar[a.rk];
+  lds_barrier();
+  const int nrow = 3 * g.nz, ncol = 2 * g.ls + g.nkx1;
+  plane_rows_fwd(A, g, T, nrow, recip_dev((unsigned)nrow));
+  // the columns of all three products at once (between them the columns kx >
+  // NKX, whose results nothing reads)
+  lds_fft<false, true, false>(A, g.pcol, ncol, recip_dev((unsigned)ncol), 3 * g.ls, T.twc);
+  // the products subtracted from CF with their derivative factors (c==0 takes
+  // (ikz, ikx, 1), all others (ikx, ikz, 1)), new CF stored, CR into the plane
+  // of the inverse transform, its de-aliased rows zero
+  double2 *I = A + 3 * g.nz * g.ls;
+  for (int e = threadIdx.x; e < g.nz * g.nkx1; e += nthr) {
+    const int zr = (int)fdiv((unsigned)e, g.f_nkx1), kx = e - zr * g.nkx1;
+    if (zr > g.nkz && zr < g.nz - g.nkz) I[inv_row(T, zr) * g.ls + kx] = make_double2(0.0, 0.0);
+  }
+  auto finish = [&](int m, const Mode &md) {
+    const int zr = kz_row(g, md.kzp);
+    const long long o = (long long)J * g.pf + m;
+    double2 acc = md.cf;
+    const double2 *col = A + 3 * T.posz[zr] * g.ls + md.kxi;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const double2 s0 = col[p * g.ls];
+      const double2 s = make_double2(div_by_recip(s0.x, g.dnz, g.rnz), div_by_recip(s0.y, g.dnz, g.rnz));
+      acc = csub(acc, (p == 2) ? s : cmul_ik((p == (c == 0 ? 0 : 1)) ? md.kz : md.kx, s));
+    }
+    ((c < 3) ? a.cf[c] : a.cfth + (c - 3) * a.cfs)[o] = acc;
+    I[inv_row(T, zr) * g.ls + md.kxi] = make_double2(md.cr.x + T5 * acc.x, md.cr.y + T5 * acc.y);
+  };
+  if ((int)threadIdx.x < g.pf) finish(threadIdx.x, md0);
+  for (int m = threadIdx.x + nthr; m < g.pf; m += nthr) finish(m, form_mode(m, load_mode(m)));
+  lds_barrier();
+  plane_cols_inv(I, g, T);
+  plane_rows_inv(I, g, T);
+  double2 *dst = reinterpret_cast<double2 *>(static_cast<double *>(a.rphys) + (long long)c * a.fs + (long long)J * g.pp);
+  for (int e = threadIdx.x; e < slots; e += nthr) {
+    const int z = (int)fdiv((unsigned)e, g.f_lw);
+    dst[e] = I[inv_slot(g, T, z, e - z * g.lw)];
+  }
+}
+template <bool SGS>
+__global__ void __launch_bounds__(kNlSmallThreads, 4) k_nonlinear_small(StepArgs a) {
+  extern __shared__ double2 smem[];
+  nonlinear_small<SGS>(a, smem);
+}
+__global__ void __launch_bounds__(kNlSmallThreads, 4) k_nonlinear_small_b(const StepArgs *__restrict__ av) {
+  extern __shared__ double2 smem[];
+  nonlinear_small<false>(av[blockIdx.z], smem);
+}
+
 // The nonlinear pass for planes too large for LDS (FP64, no LES): the same
 // terms in the same order as nonlinear_pass's LDS variant, with the
 // transforms staged through the LDS buffer `buf` (gp_rows_fwd and its
@@ -1967,6 +2264,18 @@ static NlKernel nonlinear_kernel(const Ctx &c) {
     return {(const void *)k_nonlinear32<false, kMaxQ>, (const void *)k_nonlinear32_b<false, kMaxQ>, c.plane_threads,
             (unsigned)c.lds_bytes32};
   }
+  // Small planes take their three products side by side, up to the size where
+  // a plane fills its block by itself (whole steps, this form against the
+  // other: 144 x 257 x 12, 864 values, 270 and 279 us; 256 x 101 x 8, 1024
+  // values, slower by 4%) and except where the x rows run in registers (64 x
+  // 150 x 32: 288 and 251 us).  The block size is this kernel's own.
+  const int slots = c.g.nz * c.g.lw;
+  if (slots <= kNlSmallSlots && !c.reg_rows) {
+    const int thr = slots <= 256 ? 128 : kNlSmallThreads;
+    const unsigned small = (unsigned)(c.lds_bytes + 3 * c.g.nz * c.g.ls * (int)sizeof(double2));
+    return {c.les ? (const void *)k_nonlinear_small<true> : (const void *)k_nonlinear_small<false>,
+            c.les ? nullptr : (const void *)k_nonlinear_small_b, thr, small};
+  }
   const bool half = c.plane_threads <= 512;  // the LDS variant's 512-thread instantiation
   const unsigned lds = (unsigned)c.lds_bytes;
   if (c.les) {  // FP64 only; the LES kernels have no batched forms
@@ -2762,6 +3071,8 @@ hipError_t prepare_step_kernels(Ctx &c) {
                        (const void *)k_nonlinear32<true, kNlRegQ>,  (const void *)k_nonlinear32<false, kMaxQ>,
                        (const void *)k_nonlinear_b<true, kNlRegQ>,  (const void *)k_nonlinear_b<false, kMaxQ>,
                        (const void *)k_nonlinear32_b<true, kNlRegQ>, (const void *)k_nonlinear32_b<false, kMaxQ>,
+                       (const void *)k_nonlinear_small<true>,       (const void *)k_nonlinear_small<false>,
+                       (const void *)k_nonlinear_small_b,
                        (const void *)k_rem_div_mixed,               (const void *)k_rem_div_mixed_b,
                        (const void *)k_rem_div_mixed_cn};
   for (const void *fn : fns) {
