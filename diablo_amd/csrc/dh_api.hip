@@ -329,7 +329,9 @@ int dh_create(const dh_params *p, dh_ctx **out) {
   ACHK(dalloc(&c.rphys, ph_elems * c.nfields));
   if (c.gp) {
     c.gp_slot = (long long)g.nz * g.nkx1 + g.pf;  // the plane between passes, then the accumulators
-    ACHK(dalloc(&c.gp_scratch, 2 * (size_t)kGpSlots * (size_t)c.gp_slot));
+    c.gp_elems = 2LL * kGpSlots * c.gp_slot;
+    c.pencil = g.nx <= kPencilMax && g.nz <= kPencilMax;
+    ACHK(dalloc(&c.gp_scratch, (size_t)c.gp_elems));
   }
   ACHK(dalloc(&c.rd_ta, cf_elems));
   ACHK(dalloc(&c.rd_tb, cf_elems));

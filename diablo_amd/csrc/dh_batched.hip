@@ -21,13 +21,6 @@
 
 namespace dh {
 
-// Workgroups are dealt to the 8 XCDs in turn: the index of this block when
-// XCD x takes a contiguous range of the grid's work instead.
-__device__ __forceinline__ long long xcd_range_block() {
-  const unsigned b = blockIdx.x, x = b & 7, q = gridDim.x >> 3, r = gridDim.x & 7;
-  return (long long)x * q + min(x, r) + (b >> 3);
-}
-
 // ---------------------------------------------------------------------------
 // Batched Crank-Nicolson solve.  System s, row j (0..ny-1):
 //   a_j x_{j-1} + b_j x_j + c_j x_{j+1} = d_j,
@@ -86,7 +79,7 @@ __device__ __forceinline__ void cn_solve_block(const double *__restrict__ alpha,
   // a block's row segment is one or two whole cache lines in FP64 (half of
   // that in FP32) only where nsys keeps it aligned: blocks that share a line
   // share an L2
-  const long long sys = xcd_range_block() * kCnSys + sw;
+  const long long sys = (long long)xcd_range_block() * kCnSys + sw;
   const bool live = sys < nsys;
   const long long sysc = live ? sys : nsys - 1;  // loads of idle lanes stay in bounds
   const int r0 = (w * kCnSeg + p) * R;
@@ -468,7 +461,7 @@ __global__ void __launch_bounds__(64 * CT) k_fft512_cols(const C *src, C *dst, S
   extern __shared__ double2 smraw[];
   C *tile = reinterpret_cast<C *>(smraw);
   const int c = threadIdx.x % CT, l = threadIdx.x / CT;
-  const long long col = xcd_range_block() * CT + c;
+  const long long col = (long long)xcd_range_block() * CT + c;
   const bool live = col < np * kFftK;
   const long long plane = live ? col / kFftK : 0;
   const int kx = live ? (int)(col - plane * kFftK) : 0;

@@ -211,6 +211,189 @@ __global__ void __launch_bounds__(kGpThreads, 4) k_plane_fwd_gp(PlaneArgs pa, do
   }
 }
 
+// ---------------------------------------------------------------------------
+// The transforms as pencils (FP64): Q holds the planes between the passes,
+// field f at Q + f qfs, plane j0 + jj of it at jj NZ stride.
+// ---------------------------------------------------------------------------
+struct PencilArgs {
+  Geo g;
+  PlaneBatch b;
+  double2 *q;
+  long long qfs;
+  int stride, np, nf, rows;  // planes, fields, rows per row block
+};
+
+// Fourier -> natural z rows of the kept x modes: columns k0..k0+7 of plane jj
+// of field f, unpacked (mpi.f:1562-1574).
+__global__ void __launch_bounds__(kPencilThreads, 4) k_pencil_inv_cols(PencilArgs a) {
+  extern __shared__ double2 smem[];
+  const Geo &g = a.g;
+  constexpr int CT = kPencilCols, ls = CT + 1;
+  const unsigned ntile = a.stride / CT, w = xcd_range_block();
+  const unsigned tile = w % ntile, r = w / ntile, jj = r % a.np, f = r / a.np;
+  const long long j = a.b.j0 + (long long)jj;
+  if (j < a.b.jlo[f]) return;
+  const Tables T = load_col_tables(smem + g.nz * ls, g);
+  const double2 *src = a.b.four[f] ? a.b.four[f] + j * g.pf : nullptr;
+  const int k0 = tile * CT;
+  lds_barrier();
+  gp_move<4, double2>(
+      g.nz * CT,
+      [&](int e) {
+        const int zr = e / CT, kx = k0 + e % CT;
+        int kzp = -1;
+        if (zr <= g.nkz)
+          kzp = zr;
+        else if (zr >= g.nz - g.nkz)
+          kzp = zr - (g.nz - 1 - g.nkz) + g.nkz;
+        return (kzp >= 0 && kx < g.nkx1 && src) ? src[kzp * g.nkx1 + kx] : make_double2(0.0, 0.0);
+      },
+      [&](int e, double2 v) { smem[T.posz[e / CT] * ls + e % CT] = v; });
+  lds_barrier();
+  lds_cols_inv_mirror(smem, g.pcol, CT, recip_dev(CT), ls, T.twc);
+  double2 *q = a.q + f * a.qfs + (long long)jj * g.nz * a.stride + k0;
+  for (int e = threadIdx.x; e < g.nz * CT; e += blockDim.x) q[(e / CT) * a.stride + e % CT] = smem[(e / CT) * ls + e % CT];
+}
+
+// natural z rows -> physical rows, a.rows of plane jj of field f
+__global__ void __launch_bounds__(256, 4) k_pencil_inv_rows(PencilArgs a) {
+  extern __shared__ double2 smem[];
+  const Geo &g = a.g;
+  const unsigned ng = (g.nz + a.rows - 1) / a.rows, w = xcd_range_block();
+  const unsigned grp = w % ng, r = w / ng, jj = r % a.np, f = r / a.np;
+  const long long j = a.b.j0 + (long long)jj;
+  if (j < a.b.jlo[f]) return;
+  const int r0 = grp * a.rows, nr = min(a.rows, g.nz - r0);
+  const Tables T = load_row_tables(smem + a.rows * g.ls, g);
+  const double2 *q = a.q + f * a.qfs + ((long long)jj * g.nz + r0) * a.stride;
+  gp_move<4, double2>(
+      nr * g.nkx1,
+      [&](int e) {
+        const int z = (int)fdiv((unsigned)e, g.f_nkx1);
+        return q[z * a.stride + (e - z * g.nkx1)];
+      },
+      [&](int e, double2 v) {
+        const int z = (int)fdiv((unsigned)e, g.f_nkx1);
+        smem[z * g.ls + (e - z * g.nkx1)] = v;
+      });
+  lds_barrier();
+  plane_rows_inv(smem, g, T, nr, recip_dev((unsigned)nr));
+  double2 *dst = reinterpret_cast<double2 *>(static_cast<double *>(a.b.phys[f]) + j * g.pp) + (long long)r0 * g.lw;
+  for (int e = threadIdx.x; e < nr * g.lw; e += blockDim.x) {
+    const int z = (int)fdiv((unsigned)e, g.f_lw);
+    dst[e] = smem[z * g.ls + T.posrd[e - z * g.lw]];
+  }
+}
+
+// physical rows -> x modes
+__global__ void __launch_bounds__(256, 4) k_pencil_fwd_rows(PencilArgs a) {
+  extern __shared__ double2 smem[];
+  const Geo &g = a.g;
+  const unsigned ng = (g.nz + a.rows - 1) / a.rows, w = xcd_range_block();
+  const unsigned grp = w % ng, r = w / ng, jj = r % a.np, f = r / a.np;
+  const long long j = a.b.j0 + (long long)jj;
+  const int r0 = grp * a.rows, nr = min(a.rows, g.nz - r0);
+  const Tables T = load_row_tables(smem + a.rows * g.ls, g);
+  const void *ph = (a.b.alt[f] && j >= a.b.alo[f] && j <= a.b.ahi[f]) ? a.b.alt[f] : a.b.phys[f];
+  const double2 *src = reinterpret_cast<const double2 *>(static_cast<const double *>(ph) + j * g.pp) + (long long)r0 * g.lw;
+  lds_barrier();
+  gp_move<4, double2>(
+      nr * g.lw, [&](int e) { return src[e]; },
+      [&](int e, double2 v) {
+        const int z = (int)fdiv((unsigned)e, g.f_lw);
+        smem[z * g.ls + T.posr[e - z * g.lw]] = v;
+      });
+  lds_barrier();
+  plane_rows_fwd(smem, g, T, nr, recip_dev((unsigned)nr));
+  double2 *q = a.q + f * a.qfs + ((long long)jj * g.nz + r0) * a.stride;
+  for (int e = threadIdx.x; e < nr * g.nkx1; e += blockDim.x) {
+    const int z = (int)fdiv((unsigned)e, g.f_nkx1), k = e - z * g.nkx1;
+    q[z * a.stride + k] = smem[z * g.ls + k];
+  }
+}
+
+// x modes -> Fourier, columns k0..k0+7 of plane jj of field f, packed and
+// divided by NZ (mpi.f:1529-1539)
+__global__ void __launch_bounds__(kPencilThreads, 4) k_pencil_fwd_cols(PencilArgs a) {
+  extern __shared__ double2 smem[];
+  const Geo &g = a.g;
+  constexpr int CT = kPencilCols, ls = CT + 1;
+  const unsigned ntile = a.stride / CT, w = xcd_range_block();
+  const unsigned tile = w % ntile, r = w / ntile, jj = r % a.np, f = r / a.np;
+  const long long j = a.b.j0 + (long long)jj;
+  const Tables T = load_col_tables(smem + g.nz * ls, g);
+  const int k0 = tile * CT;
+  const double2 *q = a.q + f * a.qfs + (long long)jj * g.nz * a.stride + k0;
+  gp_move<4, double2>(
+      g.nz * CT,
+      [&](int e) { return k0 + e % CT < g.nkx1 ? q[(e / CT) * a.stride + e % CT] : make_double2(0.0, 0.0); },
+      [&](int e, double2 v) { smem[(e / CT) * ls + e % CT] = v; });
+  lds_barrier();
+  lds_fft<false, true, false>(smem, g.pcol, CT, recip_dev(CT), ls, T.twc);
+  double2 *dst = const_cast<double2 *>(a.b.four[f]) + j * g.pf;
+  for (int e = threadIdx.x; e < g.nkz1 * CT; e += blockDim.x) {
+    const int kzp = e / CT, c = e % CT;
+    if (k0 + c < g.nkx1) {
+      const double2 v = smem[T.posz[kz_row(g, kzp)] * ls + c];
+      dst[kzp * g.nkx1 + k0 + c] = make_double2(div_by_recip(v.x, g.dnz, g.rnz), div_by_recip(v.y, g.dnz, g.rnz));
+    }
+  }
+}
+
+// rows of a row block: about 2048 values
+int pencil_rows(const Geo &g) { return max(1, 2048 / g.lw); }
+
+static hipError_t pencil_rows_launch(Ctx &c, bool inv, const PencilArgs &a, hipStream_t st) {
+  const unsigned lds = (unsigned)((a.rows * c.g.ls + row_table_elems(c.g)) * sizeof(double2));
+  const unsigned blocks = (unsigned)((c.g.nz + a.rows - 1) / a.rows) * a.np * a.nf;
+  if (inv)
+    hipLaunchKernelGGL(k_pencil_inv_rows, dim3(blocks), dim3(256), lds, st, a);
+  else
+    hipLaunchKernelGGL(k_pencil_fwd_rows, dim3(blocks), dim3(256), lds, st, a);
+  return hipGetLastError();
+}
+static hipError_t pencil_cols_launch(Ctx &c, bool inv, const PencilArgs &a, hipStream_t st) {
+  const unsigned lds = (unsigned)((c.g.nz * (kPencilCols + 1) + col_table_elems(c.g)) * sizeof(double2));
+  const unsigned blocks = (unsigned)(a.stride / kPencilCols) * a.np * a.nf;
+  if (inv)
+    hipLaunchKernelGGL(k_pencil_inv_cols, dim3(blocks), dim3(kPencilThreads), lds, st, a);
+  else
+    hipLaunchKernelGGL(k_pencil_fwd_cols, dim3(blocks), dim3(kPencilThreads), lds, st, a);
+  return hipGetLastError();
+}
+
+// grid.x planes of grid.y fields, as many planes at a time as the scratch
+// holds
+template <bool INV>
+static hipError_t plane_pencil(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b) {
+  if (c.recording) return hipErrorNotSupported;  // no batched forms
+  PencilArgs a{c.g, b, c.gp_scratch, 0, pencil_stride(c.g), 0, (int)grid.y, pencil_rows(c.g)};
+  const long long plane = (long long)c.g.nz * a.stride;
+  const int chunk = (int)min((long long)grid.x, c.gp_elems / (plane * a.nf));
+  for (int p0 = 0; p0 < (int)grid.x; p0 += chunk) {
+    a.np = min(chunk, (int)grid.x - p0);
+    a.b.j0 = b.j0 + p0;
+    a.qfs = a.np * plane;
+    hipError_t e = INV ? pencil_cols_launch(c, true, a, st) : pencil_rows_launch(c, false, a, st);
+    if (e == hipSuccess) e = INV ? pencil_rows_launch(c, true, a, st) : pencil_cols_launch(c, false, a, st);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+// The row pass of the inverse transform alone: planes j0..j0+np-1 of nf
+// physical fields (field f's below jlo[f] left alone) from Q.
+hipError_t launch_pencil_rows_inv(Ctx &c, double2 *q, long long qfs, double *const *phys, const int *jlo, int nf, int j0,
+                                  int np, hipStream_t st) {
+  PencilArgs a{c.g, PlaneBatch{}, q, qfs, pencil_stride(c.g), np, nf, pencil_rows(c.g)};
+  for (int f = 0; f < nf; ++f) {
+    a.b.phys[f] = phys[f];
+    a.b.jlo[f] = jlo[f];
+  }
+  a.b.j0 = j0;
+  return pencil_rows_launch(c, true, a, st);
+}
+
 static hipError_t set_lds(const void *fn, int bytes) {
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
@@ -235,7 +418,7 @@ static hipError_t plane_gp(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &
 template <class C>
 static hipError_t plane_inv(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b) {
   if constexpr (sizeof(C) == sizeof(double2))
-    if (c.gp) return plane_gp<true>(c, grid, st, b);
+    if (c.gp) return c.pencil ? plane_pencil<true>(c, grid, st, b) : plane_gp<true>(c, grid, st, b);
   const PlaneArgs pa{c.g, b};
   const unsigned lds = lds_bytes_of<C>(c);
   if (c.reg_rows)
@@ -247,7 +430,7 @@ static hipError_t plane_inv(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch 
 template <class C>
 static hipError_t plane_fwd(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b) {
   if constexpr (sizeof(C) == sizeof(double2))
-    if (c.gp) return plane_gp<false>(c, grid, st, b);
+    if (c.gp) return c.pencil ? plane_pencil<false>(c, grid, st, b) : plane_gp<false>(c, grid, st, b);
   const PlaneArgs pa{c.g, b};
   const unsigned lds = lds_bytes_of<C>(c);
   if (c.reg_rows)
@@ -415,6 +598,9 @@ static hipError_t set_lds_plane() {
 hipError_t prepare_fft_kernels(Ctx &c) {
   if (c.lds_bytes > kLdsMax && !c.gp) return hipErrorInvalidValue;
   hipError_t e;
+  for (const void *fn : {(const void *)k_pencil_inv_cols, (const void *)k_pencil_inv_rows,
+                         (const void *)k_pencil_fwd_rows, (const void *)k_pencil_fwd_cols})
+    if ((e = set_lds(fn, kLdsMax)) != hipSuccess) return e;
   if ((e = set_lds((const void *)k_plane_inv_gp, kGpLds)) != hipSuccess) return e;
   if ((e = set_lds((const void *)k_plane_fwd_gp, kGpLds)) != hipSuccess) return e;
   if ((e = set_lds_plane<true, double2>()) != hipSuccess) return e;

@@ -979,4 +979,68 @@ __device__ void gp_rows_inv(const C *Q, const Geo &g, const TablesT<C> &T, C *bu
   }
 }
 
+// ---------------------------------------------------------------------------
+// Pencils: the passes of a transform as launches of their own over many
+// planes, each block on a few whole rows or on kPencilCols whole columns of a
+// plane, so that several blocks share a CU's LDS and a plane of any size up
+// to kPencilMax keeps every pass's loads and stores in the open.  Between the
+// passes a plane is NZ rows of the NKX + 1 kept x modes, padded to a multiple
+// of kPencilCols (pencil_stride), in device memory.
+// ---------------------------------------------------------------------------
+// The x transform's tables in LDS at p (row_table_elems values), and the z
+// transform's (col_table_elems); the caller's barrier completes them.
+__host__ __device__ inline int row_table_elems(const Geo &g) { return 2 * g.lw + 1 + (2 * g.lw + 3) / 4; }
+__host__ __device__ inline int col_table_elems(const Geo &g) { return g.nz + (g.nz + 3) / 4; }
+__device__ __forceinline__ Tables load_row_tables(double2 *p, const Geo &g) {
+  Tables t{};
+  t.twr = p;
+  t.twx = p + g.lw;
+  t.posr = reinterpret_cast<int *>(p + 2 * g.lw + 1);
+  t.posrd = t.posr + g.lw;
+  for (int i = threadIdx.x; i <= g.lw; i += blockDim.x) {
+    t.twx[i] = g.tw_real[i];
+    if (i < g.lw) {
+      t.twr[i] = g.tw_row[i];
+      t.posr[i] = g.posr[i];
+      t.posrd[i] = g.posrd[i];
+    }
+  }
+  return t;
+}
+__device__ __forceinline__ Tables load_col_tables(double2 *p, const Geo &g) {
+  Tables t{};
+  t.twc = p;
+  t.posz = reinterpret_cast<int *>(p + g.nz);
+  for (int i = threadIdx.x; i < g.nz; i += blockDim.x) {
+    t.twc[i] = g.tw_col[i];
+    t.posz[i] = g.posz[i];
+  }
+  return t;
+}
+
+// Inverse column transforms from the order in which the forward ones (by
+// decimation in frequency) leave their rows, row of index k at posz[k], to
+// natural rows: the forward stages mirrored, last one first.
+template <class C>
+__device__ void lds_cols_inv_mirror(C *A, const FftPlan &pl, int ntrans, unsigned long long fnt, int ls, const C *tw) {
+#pragma unroll 1
+  for (int s = pl.nst - 1; s >= 0; --s) {
+    const FftStage &st = pl.dif[s];
+    switch (st.R) {
+      case 16: fft_stage<16, true, true, true>(A, st, pl.n, ntrans, fnt, ls, tw); break;
+      case 8: fft_stage<8, true, true, true>(A, st, pl.n, ntrans, fnt, ls, tw); break;
+      case 4: fft_stage<4, true, true, true>(A, st, pl.n, ntrans, fnt, ls, tw); break;
+      case 3: fft_stage<3, true, true, true>(A, st, pl.n, ntrans, fnt, ls, tw); break;
+      default: fft_stage<2, true, true, true>(A, st, pl.n, ntrans, fnt, ls, tw); break;
+    }
+  }
+}
+
+// Workgroups are dealt to the 8 XCDs in turn: the index of this block when
+// XCD x takes a contiguous range of the grid's work instead.
+__device__ __forceinline__ unsigned xcd_range_block() {
+  const unsigned b = blockIdx.x, x = b & 7, q = gridDim.x >> 3, r = gridDim.x & 7;
+  return x * q + min(x, r) + (b >> 3);
+}
+
 }  // namespace dh

@@ -205,6 +205,8 @@ struct Ctx {
   // modes, then the nonlinear pass's accumulators of the PF modes)
   bool gp = false;
   double2 *gp_scratch = nullptr;
+  bool pencil = false;          // large planes run as pencils (NX, NZ <= kPencilMax)
+  long long gp_elems = 0;       // complex values of gp_scratch
   long long gp_slot = 0;
 };
 inline double2 *gp_base(const Ctx &c, hipStream_t st) {
@@ -221,6 +223,19 @@ __host__ __device__ inline int gp_table_elems(const Geo &g) {
   return (2 * g.lw + g.nz + 1) + ((2 * g.lw + 2 * g.nz) * (int)sizeof(int) + 15) / 16;
 }
 __host__ __device__ inline int gp_stage_elems(const Geo &g) { return kGpLds / 16 - gp_table_elems(g); }
+// Pencils (dh_fft_dev.h): columns of a column block (128 B of every row), its
+// threads, the largest NX and NZ, and the padded row of kept x modes.
+constexpr int kPencilCols = 8;
+constexpr int kPencilThreads = 512;
+// (a column block of the nonlinear pass at NZ = 512 fills the LDS, 150 KB; longer
+// rows and columns run on the persistent kernels above, planes that fit LDS on
+// the plane kernels: 128 x 129 x 128 takes 1.31 ms for two steps there and
+// 1.95 as pencils)
+constexpr int kPencilMax = 512;
+__host__ __device__ inline int pencil_stride(const Geo &g) {
+  return (g.nkx1 + kPencilCols - 1) / kPencilCols * kPencilCols;
+}
+
 // feature slots of the learned closure: 0..5 the network's inputs, 6..11
 // S11, S22, S33, S12, S13, S23 at GY, 12 |S| at GY
 constexpr int kLesFeat = 13;
@@ -286,6 +301,8 @@ template <class C>
 inline int lds_bytes_of(const Ctx &c) {
   return sizeof(C) == sizeof(double2) ? c.lds_bytes : c.lds_bytes32;
 }
+hipError_t launch_pencil_rows_inv(Ctx &c, double2 *q, long long qfs, double *const *phys, const int *jlo, int nf, int j0,
+                                  int np, hipStream_t st);
 hipError_t launch_fft_to_phys(Ctx &c, const double2 *four, double *phys, int nplanes);
 hipError_t launch_stats(Ctx &c, double *out_dev);  // profiles of dh_save_stats into out_dev
 hipError_t launch_fft_to_four(Ctx &c, const double *phys, double2 *four, int nplanes);

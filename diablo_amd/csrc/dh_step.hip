@@ -607,14 +607,20 @@ struct RkRow {
   double ey0, ey1, ey2, rey0, rey1, rey2;  // weights of C(J+1)-C(J), C(J)-C(J-1) and the outer divisor
   double dy, rdy;
 };
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ double uniform(double x) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
 __device__ __forceinline__ RkRow rk_row(const StepArgs &a, int c, int J) {
   const Geo &g = a.g;
   RkRow r;
   const double hb = a.clk->h_bar[a.rk];
-  r.T3 = a.clk->zeta_bar[a.rk] * hb;
+  r.T3 = uniform(a.clk->zeta_bar[a.rk] * hb);
   r.T4 = hb;
-  r.T5 = a.clk->beta_bar[a.rk] * hb;
+  r.T5 = uniform(a.clk->beta_bar[a.rk] * hb);
   r.coefv = (c < 3) ? (a.nu * hb / 2.0) * a.nu_v_scale : ((a.nu * hb / 2.0) / a.pr[c - 3]) * a.nu_v_scale;
+  r.coefv = uniform(r.coefv);
   const bool v = c == 1;
   r.ey0 = v ? g.dyf[J] : g.dy[J + 1];
   r.ey1 = v ? g.dyf[J - 1] : g.dy[J];
@@ -892,6 +898,161 @@ __global__ void __launch_bounds__(kNlSmallThreads, 4) k_nonlinear_small(StepArgs
 __global__ void __launch_bounds__(kNlSmallThreads, 4) k_nonlinear_small_b(const StepArgs *__restrict__ av) {
   extern __shared__ double2 smem[];
   nonlinear_small<false>(av[blockIdx.z], smem);
+}
+
+// ---------------------------------------------------------------------------
+// The nonlinear pass of large planes as pencils (FP64, no LES).  Per component
+// the products enter the z transform as two arrays of x modes: Z, the product
+// that takes ikz, and M = ikx X + Y, the product that takes ikx and the y flux
+// (KX is constant along z, so they share a transform).  Of the velocity
+// components' nine products eight differ (U1 U3 serves U1 and U3), and all are
+// formed from one reading of a row's samples.
+//   k_pencil_products  row blocks: products, x transforms, Z and M of every
+//                      component to Q
+//   k_pencil_combine   column blocks: z transforms of Z and M, CF and the RK
+//                      combination mode by mode, the inverse z transform of
+//                      CR over Z's place
+//   k_pencil_inv_rows  (dh_fft.hip) the inverse x transform to R
+//
+// What bounds it: per 96 planes of 256 x 256 the products take 156 us (the
+// LDS stages of eight row transforms per row; 0.36 GB from and to memory),
+// the combination 204 (0.58 GB; the modes' loads, 16 waves on a CU) and the
+// inverse rows 67 (0.23 GB).  One block per CU that keeps a plane's transform
+// to itself (nonlinear_pass_gp), with the plane and CF's accumulators passing
+// through memory between all its passes, took 1.74 ms a substep at 256 x 193 x
+// 256 where these take 0.85.  Loading three modes per thread ahead of the
+// tile spilled and was slower (297 us for 204); four columns per block: 215.
+// ---------------------------------------------------------------------------
+struct PencilStep {
+  double2 *q;         // [2 (c - c0) + (0: Z, 1: M)][plane][NZ][stride]
+  long long qfs;      // one array
+  int stride, np, j0, rows;
+};
+
+// Rows of plane J of the products of U1..U3 (N = 8) or of scalar c (N = 3).
+template <int N>
+__global__ void __launch_bounds__(kPencilThreads, 4) k_pencil_products(StepArgs a, PencilStep s) {
+  extern __shared__ double2 smem[];
+  const Geo &g = a.g;
+  // planes inner: a row block's planes J, J+1, ... follow each other on an
+  // XCD, whose L2 keeps the rows they share
+  const unsigned w = xcd_range_block();
+  const int jj = w % s.np, J = s.j0 + jj, r0 = (w / s.np) * s.rows;
+  const int c = a.c0;
+  if (N == 3 && (J < a.jstart_th[c - 3] || J > a.jend_th[c - 3])) return;
+  if (N == 8 && (J < 2 || J > g.ny)) return;
+  const int nr = min(s.rows, g.nz - r0);
+  const int e = threadIdx.x, zl = (int)fdiv((unsigned)e, g.f_lw), xp = e - zl * g.lw;
+  const bool in = zl < nr;
+  const double *up = static_cast<const double *>(a.uphys);
+  const long long off = (long long)(r0 + (in ? zl : 0)) * g.nx + 2 * xp;
+  auto smp = [&](int f, int j) { return *reinterpret_cast<const double2 *>(up + f * a.fs + (long long)j * g.pp + off); };
+  const Tables T = load_row_tables(smem + N * s.rows * g.ls, g);
+  double2 v[N];
+  if constexpr (N == 8) {
+    const Prod<double2> pi = make_prod<double2>(a, 1, 0, J), py = make_prod<double2>(a, 0, 2, J),
+                        pv = make_prod<double2>(a, 1, 2, J);
+    const double2 u1p = smp(0, J + 1), u10 = smp(0, J), u1m = smp(0, J - 1);
+    const double2 u3p = smp(2, J + 1), u30 = smp(2, J), u3m = smp(2, J - 1);
+    const double2 u2p = smp(1, J + 1), u20 = smp(1, J), u2m = smp(1, J - 1);
+    v[0] = eval_raw<0, double2>(pi, ProdRaw<0, double2>{{u30, u10}});
+    v[1] = eval_raw<1, double2>(pi, ProdRaw<1, double2>{{u10}});
+    v[2] = eval_raw<1, double2>(pi, ProdRaw<1, double2>{{u30}});
+    v[3] = eval_raw<3, double2>(pi, ProdRaw<3, double2>{{u10, u1m, u20}});
+    v[4] = eval_raw<3, double2>(pi, ProdRaw<3, double2>{{u30, u3m, u20}});
+    v[5] = eval_raw<2, double2>(py, ProdRaw<2, double2>{{u1p, u10, u1m, u2p, u20}});
+    v[6] = eval_raw<2, double2>(py, ProdRaw<2, double2>{{u3p, u30, u3m, u2p, u20}});
+    v[7] = eval_raw<4, double2>(pv, ProdRaw<4, double2>{{u2p, u20, u2m}});
+  } else {
+    const Prod<double2> py = make_prod<double2>(a, c, 2, J);
+    const double2 tp = smp(c, J + 1), t0 = smp(c, J), tm = smp(c, J - 1), u2p = smp(1, J + 1), u20 = smp(1, J);
+    v[0] = eval_raw<0, double2>(py, ProdRaw<0, double2>{{t0, smp(0, J)}});
+    v[1] = eval_raw<0, double2>(py, ProdRaw<0, double2>{{t0, smp(2, J)}});
+    v[2] = eval_raw<2, double2>(py, ProdRaw<2, double2>{{tp, t0, tm, u2p, u20}});
+  }
+  lds_barrier();
+  if (in) {
+#pragma unroll
+    for (int p = 0; p < N; ++p) smem[(p * nr + zl) * g.ls + T.posr[xp]] = v[p];
+  }
+  lds_barrier();
+  plane_rows_fwd(smem, g, T, N * nr, recip_dev((unsigned)(N * nr)));
+  double2 *q = s.q + ((long long)jj * g.nz + r0) * s.stride;
+  for (int i = threadIdx.x; i < nr * g.nkx1; i += blockDim.x) {
+    const int z = (int)fdiv((unsigned)i, g.f_nkx1), k = i - z * g.nkx1;
+    const double kx = g.kx[k];
+    auto F = [&](int p) { return smem[(p * nr + z) * g.ls + k]; };
+    double2 *o = q + z * s.stride + k;
+    if constexpr (N == 8) {
+      const double2 f13 = F(0);
+      o[0] = f13;
+      o[s.qfs] = cadd(cmul_ik(kx, F(1)), F(5));
+      o[2 * s.qfs] = F(4);
+      o[3 * s.qfs] = cadd(cmul_ik(kx, F(3)), F(7));
+      o[4 * s.qfs] = F(2);
+      o[5 * s.qfs] = cadd(cmul_ik(kx, f13), F(6));
+    } else {
+      o[0] = F(1);
+      o[s.qfs] = cadd(cmul_ik(kx, F(0)), F(2));
+    }
+  }
+}
+
+// Columns k0..k0+7 of plane J of component a.c0 + ic.
+__global__ void __launch_bounds__(kPencilThreads, 4) k_pencil_combine(StepArgs a, PencilStep s) {
+  extern __shared__ double2 smem[];
+  const Geo &g = a.g;
+  constexpr int CT = kPencilCols, ls = 2 * CT + 1;
+  const unsigned ntile = s.stride / CT, w = xcd_range_block();
+  const unsigned tile = w % ntile, r = w / ntile, jj = r % s.np, ic = r / s.np;
+  const int J = s.j0 + (int)jj, c = a.c0 + (int)ic, k0 = tile * CT;
+  int jlo = 2, jhi = g.ny;
+  if (c >= 3) {
+    jlo = a.jstart_th[c - 3];
+    jhi = a.jend_th[c - 3];
+  }
+  if (J < jlo || J > jhi) return;
+  const Tables T = load_col_tables(smem + g.nz * ls, g);
+  double2 *q = s.q + 2 * ic * s.qfs + (long long)jj * g.nz * s.stride + k0;
+  gp_move<4, double2>(
+      g.nz * 2 * CT,
+      [&](int e) {
+        const int j = e % CT, arr = (e / CT) & 1, z = e / (2 * CT);
+        return k0 + j < g.nkx1 ? q[arr * s.qfs + z * s.stride + j] : make_double2(0.0, 0.0);
+      },
+      [&](int e, double2 v) { smem[(e / (2 * CT)) * ls + e % (2 * CT)] = v; });
+  lds_barrier();
+  lds_fft<false, true, false>(smem, g.pcol, 2 * CT, recip_dev(2 * CT), ls, T.twc);
+  const RkRow rr = rk_row(a, c, J);
+  double2 *CF = (c < 3) ? a.cf[c] : a.cfth + (c - 3) * a.cfs;
+  // CR of each mode goes over its Z value, which nothing else reads; the
+  // de-aliased rows are cleared
+  for (int e = threadIdx.x; e < g.nz * CT; e += blockDim.x) {
+    const int zr = e / CT;
+    if (zr > g.nkz && zr < g.nz - g.nkz) smem[T.posz[zr] * ls + e % CT] = make_double2(0.0, 0.0);
+  }
+#pragma unroll 1
+  for (int e = threadIdx.x; e < g.nkz1 * CT; e += blockDim.x) {
+    const int kzp = e / CT, j = e % CT, kx = k0 + j;
+    if (kx >= g.nkx1) continue;
+    const long long o = (long long)J * g.pf + kzp * g.nkx1 + kx;
+    const RkMode md = rk_load(a, c, o);
+    double2 x0, x1;
+    cf_load(a, c, o, x0, x1);
+    const double kxv = g.kx[kx], kzv = g.kz[kzp];
+    const bool mean = kx == 0 && kzp == 0;
+    double2 acc = cf_terms(a, c, J, g.kx2[kx] + g.kz2[kzp], mean, o, md.c0, x0, x1);
+    const double2 cr = rk_combine<false>(a, rr, c, (c == 0) ? kxv : kzv, mean, md);
+    double2 *sl = smem + T.posz[kz_row(g, kzp)] * ls + j;
+    const double2 zv = make_double2(div_by_recip(sl[0].x, g.dnz, g.rnz), div_by_recip(sl[0].y, g.dnz, g.rnz));
+    const double2 mv = make_double2(div_by_recip(sl[CT].x, g.dnz, g.rnz), div_by_recip(sl[CT].y, g.dnz, g.rnz));
+    acc = csub(csub(acc, cmul_ik(kzv, zv)), mv);
+    CF[o] = acc;
+    sl[0] = make_double2(cr.x + rr.T5 * acc.x, cr.y + rr.T5 * acc.y);
+  }
+  lds_barrier();
+  lds_cols_inv_mirror(smem, g.pcol, CT, recip_dev(CT), ls, T.twc);
+  for (int e = threadIdx.x; e < g.nz * CT; e += blockDim.x) q[(e / CT) * s.stride + e % CT] = smem[(e / CT) * ls + e % CT];
 }
 
 // The nonlinear pass for planes too large for LDS (FP64, no LES): the same
@@ -2303,6 +2464,49 @@ static void nonlinear_rows(const Ctx &c, int c0, int c1, int &jlo, int &jhi) {
   }
 }
 
+// The nonlinear pass of fields c0..c1-1 as pencils, as many planes at a time
+// as the scratch holds arrays for (about even parts).
+static hipError_t launch_nonlinear_pencil(Ctx &c, StepArgs a, int c0, int c1, int jlo, int jhi, hipStream_t st) {
+  if (c.recording) return hipErrorNotSupported;
+  const Geo &g = c.g;
+  const int nf = c1 - c0, np = jhi - jlo + 1;
+  PencilStep s{c.gp_scratch, 0, pencil_stride(g), 0, 0, max(1, kPencilThreads / g.lw)};
+  const long long plane = (long long)g.nz * s.stride;
+  const int most = (int)min((long long)np, c.gp_elems / (2 * nf * plane));
+  const int parts = (np + most - 1) / most, chunk = (np + parts - 1) / parts;
+  const unsigned groups = (unsigned)((g.nz + s.rows - 1) / s.rows);
+  const unsigned lds_col = (unsigned)((g.nz * (2 * kPencilCols + 1) + col_table_elems(g)) * sizeof(double2));
+  for (int j = jlo; j <= jhi; j += chunk) {
+    s.j0 = j;
+    s.np = min(chunk, jhi - j + 1);
+    s.qfs = s.np * plane;
+    for (int f = c0; f < c1; f = f < 3 ? 3 : f + 1) {  // U1..U3 together, scalars one by one
+      StepArgs b = a;
+      PencilStep t = s;
+      b.c0 = f;
+      t.q = s.q + 2 * (f - c0) * s.qfs;
+      const int n = f < 3 ? 8 : 3;
+      const unsigned lds = (unsigned)((n * s.rows * g.ls + row_table_elems(g)) * sizeof(double2));
+      if (n == 8)
+        hipLaunchKernelGGL(k_pencil_products<8>, dim3(groups * s.np), dim3(kPencilThreads), lds, st, b, t);
+      else
+        hipLaunchKernelGGL(k_pencil_products<3>, dim3(groups * s.np), dim3(kPencilThreads), lds, st, b, t);
+    }
+    a.c0 = c0;
+    hipLaunchKernelGGL(k_pencil_combine, dim3((unsigned)(s.stride / kPencilCols) * s.np * nf), dim3(kPencilThreads),
+                       lds_col, st, a, s);
+    double *phys[kMaxFields];
+    int lo[kMaxFields];
+    for (int f = c0; f < c1; ++f) {
+      phys[f - c0] = c.rphys + f * a.fs;
+      lo[f - c0] = f < 3 ? 2 : c.jstart_th[f - 3];
+    }
+    const hipError_t e = launch_pencil_rows_inv(c, s.q, 2 * s.qfs, phys, lo, nf, s.j0, s.np, st);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 static hipError_t launch_nonlinear_range(Ctx &c, int rk, int c0, int c1, hipStream_t st) {
   if (c1 <= c0) return hipSuccess;
   StepArgs a = make_step_args(c, rk);
@@ -2312,6 +2516,7 @@ static hipError_t launch_nonlinear_range(Ctx &c, int rk, int c0, int c1, hipStre
   a.c0 = c0;
   a.j0 = jlo;
   const dim3 grid(jhi - jlo + 1, c1 - c0);
+  if (c.pencil) return launch_nonlinear_pencil(c, a, c0, c1, jlo, jhi, st);
   if (c.gp) {  // planes beyond LDS (FP64, no LES)
     if (c.recording) return hipErrorNotSupported;
     double2 *gp = gp_base(c, st);
@@ -2332,7 +2537,7 @@ static hipError_t launch_nonlinear_range(Ctx &c, int rk, int c0, int c1, hipStre
 // (config 1: 0.638 ms per step flat against 0.657 with the branch).  The
 // large-plane kernels keep the branch (256 x 193 x 256: 7.2 ms per step
 // against 7.55 flat).
-static bool flat_substep(const Ctx &c) { return !c.gp; }
+static bool flat_substep(const Ctx &c) { return !c.gp || c.pencil; }
 
 
 static hipError_t launch_nonlinear(Ctx &c, int rk) { return launch_nonlinear_range(c, rk, 0, c.nfields, c.stream); }
@@ -3072,7 +3277,8 @@ hipError_t prepare_step_kernels(Ctx &c) {
                        (const void *)k_nonlinear_b<true, kNlRegQ>,  (const void *)k_nonlinear_b<false, kMaxQ>,
                        (const void *)k_nonlinear32_b<true, kNlRegQ>, (const void *)k_nonlinear32_b<false, kMaxQ>,
                        (const void *)k_nonlinear_small<true>,       (const void *)k_nonlinear_small<false>,
-                       (const void *)k_nonlinear_small_b,
+                       (const void *)k_nonlinear_small_b,           (const void *)k_pencil_products<8>,
+                       (const void *)k_pencil_products<3>,          (const void *)k_pencil_combine,
                        (const void *)k_rem_div_mixed,               (const void *)k_rem_div_mixed_b,
                        (const void *)k_rem_div_mixed_cn};
   for (const void *fn : fns) {
