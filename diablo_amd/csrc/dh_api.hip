@@ -919,11 +919,10 @@ int dh_autotune(dh_ctx *h, int32_t nsteps, int32_t *chosen) {
 // three substeps, TIME += DELTA_T; the end of one step and the start of the
 // next share one launch.
 static int enqueue_steps(Ctx &c, int nsteps) {
-  HIPCHK(launch_step_boundary(c, false, true));
   for (int s = 0; s < nsteps; ++s) {
     // the boundary into the next step (or the end of the last) rides in the
     // last substep's REM_DIV launch
-    for (int rk = 0; rk < 2; ++rk) HIPCHK(launch_substep(c, rk));
+    for (int rk = 0; rk < 2; ++rk) HIPCHK(launch_substep(c, rk, 0, 0, s == 0 && rk == 0));
     HIPCHK(launch_substep(c, 2, 1, s + 1 < nsteps ? 1 : 0));
   }
   return DH_OK;

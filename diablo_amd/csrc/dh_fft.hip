@@ -30,9 +30,23 @@ struct PlaneBatch {
   int drop_mean;
 };
 
+// What one thread of a launch does beside it, as nothing of the launch reads
+// the clock: an inverse opens a step (TIME_STEP += 1), a forward after the
+// solve sets COURANT's DELTA_T.  A launch of one thread takes 4.6 us.
+struct ClockDuty {
+  CourantArgs courant;  // clk null: none
+  Clock *tick;
+};
+__device__ __forceinline__ void clock_duty(const ClockDuty &d) {
+  if (blockIdx.x != 0 || blockIdx.y != 0 || threadIdx.x != 0) return;
+  if (d.tick) d.tick->time_step += 1;
+  if (d.courant.clk) courant_dt_body(d.courant.clk, d.courant.dt_cap, d.courant.variable_dt, d.courant.update_dt);
+}
+
 struct PlaneArgs {
   Geo g;
   PlaneBatch b;
+  ClockDuty duty;
 };
 
 // Fourier -> physical for plane j of field f.  A: the plane in LDS, T: the
@@ -114,6 +128,7 @@ __device__ __forceinline__ void plane_fwd_body(const Geo &g, const PlaneBatch &b
 template <bool REG, class C>
 __global__ void __launch_bounds__(1024) k_plane_inv(PlaneArgs pa) {
   extern __shared__ double2 smem[];
+  clock_duty(pa.duty);
   C *A = reinterpret_cast<C *>(smem);
   plane_inv_body<REG, C>(pa.g, pa.b, A, load_tables(A, pa.g), blockIdx.y, pa.b.j0 + blockIdx.x);
 }
@@ -127,6 +142,7 @@ __global__ void __launch_bounds__(1024) k_plane_inv_b(const PlaneArgs *__restric
 template <bool REG, class C>
 __global__ void __launch_bounds__(1024) k_plane_fwd(PlaneArgs pa) {
   extern __shared__ double2 smem[];
+  clock_duty(pa.duty);
   C *A = reinterpret_cast<C *>(smem);
   plane_fwd_body<REG, C>(pa.g, pa.b, A, load_tables(A, pa.g), blockIdx.y, pa.b.j0 + blockIdx.x);
 }
@@ -187,6 +203,7 @@ __device__ __forceinline__ void plane_fwd_gp_body(const Geo &g, const PlaneBatch
 __global__ void __launch_bounds__(kGpThreads, 4) k_plane_inv_gp(PlaneArgs pa, double2 *gp, long long gp_slot,
                                                                 int nplanes, int nitems) {
   extern __shared__ double2 smem[];
+  clock_duty(pa.duty);
   const Tables T = load_tables_at(smem, pa.g);
   double2 *buf = smem + gp_table_elems(pa.g);
   const int stage = gp_stage_elems(pa.g);
@@ -200,6 +217,7 @@ __global__ void __launch_bounds__(kGpThreads, 4) k_plane_inv_gp(PlaneArgs pa, do
 __global__ void __launch_bounds__(kGpThreads, 4) k_plane_fwd_gp(PlaneArgs pa, double2 *gp, long long gp_slot,
                                                                 int nplanes, int nitems) {
   extern __shared__ double2 smem[];
+  clock_duty(pa.duty);
   const Tables T = load_tables_at(smem, pa.g);
   double2 *buf = smem + gp_table_elems(pa.g);
   const int stage = gp_stage_elems(pa.g);
@@ -221,6 +239,7 @@ struct PencilArgs {
   double2 *q;
   long long qfs;
   int stride, np, nf, rows;  // planes, fields, rows per row block
+  ClockDuty duty;
 };
 
 // Fourier -> natural z rows of the kept x modes: columns k0..k0+7 of plane jj
@@ -229,6 +248,7 @@ __global__ void __launch_bounds__(kPencilThreads, 4) k_pencil_inv_cols(PencilArg
   extern __shared__ double2 smem[];
   const Geo &g = a.g;
   constexpr int CT = kPencilCols, ls = CT + 1;
+  clock_duty(a.duty);
   const unsigned ntile = a.stride / CT, w = xcd_range_block();
   const unsigned tile = w % ntile, r = w / ntile, jj = r % a.np, f = r / a.np;
   const long long j = a.b.j0 + (long long)jj;
@@ -288,6 +308,7 @@ __global__ void __launch_bounds__(256, 4) k_pencil_inv_rows(PencilArgs a) {
 // physical rows -> x modes
 __global__ void __launch_bounds__(256, 4) k_pencil_fwd_rows(PencilArgs a) {
   extern __shared__ double2 smem[];
+  clock_duty(a.duty);
   const Geo &g = a.g;
   const unsigned ng = (g.nz + a.rows - 1) / a.rows, w = xcd_range_block();
   const unsigned grp = w % ng, r = w / ng, jj = r % a.np, f = r / a.np;
@@ -365,9 +386,9 @@ static hipError_t pencil_cols_launch(Ctx &c, bool inv, const PencilArgs &a, hipS
 // grid.x planes of grid.y fields, as many planes at a time as the scratch
 // holds
 template <bool INV>
-static hipError_t plane_pencil(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b) {
+static hipError_t plane_pencil(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b, const ClockDuty &duty) {
   if (c.recording) return hipErrorNotSupported;  // no batched forms
-  PencilArgs a{c.g, b, c.gp_scratch, 0, pencil_stride(c.g), 0, (int)grid.y, pencil_rows(c.g)};
+  PencilArgs a{c.g, b, c.gp_scratch, 0, pencil_stride(c.g), 0, (int)grid.y, pencil_rows(c.g), duty};
   const long long plane = (long long)c.g.nz * a.stride;
   const int chunk = (int)min((long long)grid.x, c.gp_elems / (plane * a.nf));
   for (int p0 = 0; p0 < (int)grid.x; p0 += chunk) {
@@ -377,6 +398,7 @@ static hipError_t plane_pencil(Ctx &c, dim3 grid, hipStream_t st, const PlaneBat
     hipError_t e = INV ? pencil_cols_launch(c, true, a, st) : pencil_rows_launch(c, false, a, st);
     if (e == hipSuccess) e = INV ? pencil_rows_launch(c, true, a, st) : pencil_cols_launch(c, false, a, st);
     if (e != hipSuccess) return e;
+    a.duty = ClockDuty{};  // with the first part only
   }
   return hipSuccess;
 }
@@ -385,7 +407,7 @@ static hipError_t plane_pencil(Ctx &c, dim3 grid, hipStream_t st, const PlaneBat
 // physical fields (field f's below jlo[f] left alone) from Q.
 hipError_t launch_pencil_rows_inv(Ctx &c, double2 *q, long long qfs, double *const *phys, const int *jlo, int nf, int j0,
                                   int np, hipStream_t st) {
-  PencilArgs a{c.g, PlaneBatch{}, q, qfs, pencil_stride(c.g), np, nf, pencil_rows(c.g)};
+  PencilArgs a{c.g, PlaneBatch{}, q, qfs, pencil_stride(c.g), np, nf, pencil_rows(c.g), ClockDuty{}};
   for (int f = 0; f < nf; ++f) {
     a.b.phys[f] = phys[f];
     a.b.jlo[f] = jlo[f];
@@ -403,9 +425,9 @@ static hipError_t set_lds(const void *fn, int bytes) {
 // Large planes: the persistent kernels above over grid.x planes of grid.y
 // fields, on the scratch half of the stream (the branch stream has its own).
 template <bool INV>
-static hipError_t plane_gp(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b) {
+static hipError_t plane_gp(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b, const ClockDuty &duty) {
   if (c.recording) return hipErrorNotSupported;  // no batched forms
-  PlaneArgs pa{c.g, b};
+  PlaneArgs pa{c.g, b, duty};
   double2 *gp = gp_base(c, st);
   long long slot = c.gp_slot;
   int nplanes = (int)grid.x, nitems = (int)(grid.x * grid.y);
@@ -416,10 +438,10 @@ static hipError_t plane_gp(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &
 }
 
 template <class C>
-static hipError_t plane_inv(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b) {
+static hipError_t plane_inv(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b, const ClockDuty &duty = ClockDuty{}) {
   if constexpr (sizeof(C) == sizeof(double2))
-    if (c.gp) return c.pencil ? plane_pencil<true>(c, grid, st, b) : plane_gp<true>(c, grid, st, b);
-  const PlaneArgs pa{c.g, b};
+    if (c.gp) return c.pencil ? plane_pencil<true>(c, grid, st, b, duty) : plane_gp<true>(c, grid, st, b, duty);
+  const PlaneArgs pa{c.g, b, duty};
   const unsigned lds = lds_bytes_of<C>(c);
   if (c.reg_rows)
     return klaunch(c, (const void *)k_plane_inv<true, C>, (const void *)k_plane_inv_b<true, C>, grid,
@@ -428,10 +450,10 @@ static hipError_t plane_inv(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch 
                  dim3(c.plane_threads), lds, st, pa);
 }
 template <class C>
-static hipError_t plane_fwd(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b) {
+static hipError_t plane_fwd(Ctx &c, dim3 grid, hipStream_t st, const PlaneBatch &b, const ClockDuty &duty = ClockDuty{}) {
   if constexpr (sizeof(C) == sizeof(double2))
-    if (c.gp) return c.pencil ? plane_pencil<false>(c, grid, st, b) : plane_gp<false>(c, grid, st, b);
-  const PlaneArgs pa{c.g, b};
+    if (c.gp) return c.pencil ? plane_pencil<false>(c, grid, st, b, duty) : plane_gp<false>(c, grid, st, b, duty);
+  const PlaneArgs pa{c.g, b, duty};
   const unsigned lds = lds_bytes_of<C>(c);
   if (c.reg_rows)
     return klaunch(c, (const void *)k_plane_fwd<true, C>, (const void *)k_plane_fwd_b<true, C>, grid,
@@ -490,7 +512,8 @@ hipError_t launch_fft_to_four(Ctx &c, const double *phys, double2 *four, int npl
 
 // All state fields (U1..3, TH) to the substep's physical arrays, planes
 // 0..NY+1 (channel.f:386-399).
-hipError_t launch_state_to_phys(Ctx &c) {
+// tick: the launch also opens a step.
+hipError_t launch_state_to_phys(Ctx &c, bool tick) {
   PlaneBatch b{};
   const long long fs = (long long)(c.g.ny + 2) * c.g.pp;
   const long long cfs = (long long)(c.g.ny + 2) * c.g.pf;
@@ -502,7 +525,8 @@ hipError_t launch_state_to_phys(Ctx &c) {
   b.j0 = 0;
   b.drop_mean = c.mixed;  // the mixed form keeps the plane means in FP64
   const dim3 grid(c.g.ny + 2, c.nfields);
-  return c.mixed ? plane_inv<float2>(c, grid, c.stream, b) : plane_inv<double2>(c, grid, c.stream, b);
+  const ClockDuty duty{{}, tick ? c.clock : nullptr};
+  return c.mixed ? plane_inv<float2>(c, grid, c.stream, b, duty) : plane_inv<double2>(c, grid, c.stream, b, duty);
 }
 
 // The LES substep's inverse transforms in one launch: the state fields as
@@ -553,8 +577,8 @@ hipError_t launch_state_to_four(Ctx &c) { return launch_fields_to_four(c, 0, c.n
 // (channel.f:1043-1050): the solve left planes wlo..whi of a velocity field
 // in its R array (the other planes keep the values transformed at the start
 // of the substep); velocity goes to CUN, for REM_DIV to project into CU, and
-// scalars straight to CTH.
-hipError_t launch_step_to_four(Ctx &c, int f0, int f1, hipStream_t st) {
+// scalars straight to CTH.  courant: the launch also sets COURANT's DELTA_T.
+hipError_t launch_step_to_four(Ctx &c, int f0, int f1, hipStream_t st, const CourantArgs *courant) {
   if (f1 <= f0) return hipSuccess;
   PlaneBatch b{};
   const long long fs = (long long)(c.g.ny + 2) * c.g.pp;
@@ -581,7 +605,8 @@ hipError_t launch_step_to_four(Ctx &c, int f0, int f1, hipStream_t st) {
   }
   b.j0 = 0;
   const dim3 grid(c.g.ny + 2, f1 - f0);
-  return c.mixed ? plane_fwd<float2>(c, grid, st, b) : plane_fwd<double2>(c, grid, st, b);
+  const ClockDuty duty{courant ? *courant : CourantArgs{}, nullptr};
+  return c.mixed ? plane_fwd<float2>(c, grid, st, b, duty) : plane_fwd<double2>(c, grid, st, b, duty);
 }
 
 template <bool REG, class C>

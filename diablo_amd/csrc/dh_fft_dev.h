@@ -1043,4 +1043,32 @@ __device__ __forceinline__ unsigned xcd_range_block() {
   return x * q + min(x, r) + (b >> 3);
 }
 
+// COURANT (courant.f:45-62) from the CFL minimum of the solve kernel; the
+// solve tables for the new DELTA_T are rebuilt right after by k_cn_tables.
+// One thread runs it, in a launch between the solve and REM_DIV that reads
+// nothing of the clock.
+__device__ __forceinline__ void courant_dt_body(Clock *clk, double dt_cap, int variable_dt, int update_dt) {
+  Clock &c = *clk;
+  // TEMP4 of this substep was fixed before COURANT (channel.f:80); the
+  // pressure update after REM_DIV (channel.f:1059-1065) still divides by it
+  c.h_cp = c.h_bar[2];
+  if (variable_dt && (c.time_step % update_dt) == 0) {
+    double dt = dt_cap;
+    const double m = __longlong_as_double((long long)c.cfl_min_bits);
+    if (m < dt) dt = m;
+    double DT;
+    if (dt <= 0)
+      DT = 0.0001;
+    else if (dt >= 999.)
+      DT = 999.0;
+    else
+      DT = dt;
+    c.dt = DT;
+    c.h_bar[0] = DT * (8.0 / 15.0);
+    c.h_bar[1] = DT * (2.0 / 15.0);
+    c.h_bar[2] = DT * (5.0 / 15.0);
+  }
+  c.cfl_min_bits = 0x7FF0000000000000ull;
+}
+
 }  // namespace dh

@@ -97,6 +97,12 @@ constexpr int kLdsMax = 160 * 1024;
 // one per block of the persistent large-plane kernels (kGpThreads threads).
 constexpr int kGpSlots = 256, kGpThreads = 1024;
 
+struct CourantArgs {
+  Clock *clk;
+  double dt_cap;
+  int variable_dt, update_dt;
+};
+
 // Tables of the y-implicit (Crank-Nicolson) matrices, one set per RK
 // substep and field; with LES off each matrix depends only on j, so every
 // (x,z) column of a field shares them.
@@ -306,13 +312,14 @@ hipError_t launch_pencil_rows_inv(Ctx &c, double2 *q, long long qfs, double *con
 hipError_t launch_fft_to_phys(Ctx &c, const double2 *four, double *phys, int nplanes);
 hipError_t launch_stats(Ctx &c, double *out_dev);  // profiles of dh_save_stats into out_dev
 hipError_t launch_fft_to_four(Ctx &c, const double *phys, double2 *four, int nplanes);
-hipError_t launch_state_to_phys(Ctx &c);
+hipError_t launch_state_to_phys(Ctx &c, bool tick = false);
 // LES: the state (planes 0..NY+1) and n strain fields (planes 1..NY+1) in one launch
 hipError_t launch_state_and_fields_to_phys(Ctx &c, const double2 *const *four, double *const *phys, int n,
                                            hipStream_t st);
 hipError_t launch_state_to_four(Ctx &c);
 hipError_t launch_fields_to_four(Ctx &c, int f0, int f1);
-hipError_t launch_step_to_four(Ctx &c, int f0, int f1, hipStream_t st);  // end of a substep (into CUN / CTH)
+// end of a substep (into CUN / CTH)
+hipError_t launch_step_to_four(Ctx &c, int f0, int f1, hipStream_t st, const CourantArgs *courant = nullptr);
 // ---- launchers (dh_ics.hip) ----
 hipError_t launch_apply_bc_vel(Ctx &c);
 // LES (les.f): the gated Fourier BCs that open les_chan, before the state
@@ -344,7 +351,7 @@ hipError_t launch_create_th(Ctx &c, int ic_type);
 hipError_t prepare_step_kernels(Ctx &c);
 // rk 0..2; bnd_end/bnd_begin: the step boundary after it (TIME += DELTA_T,
 // TIME_STEP += 1), done within REM_DIV's launch
-hipError_t launch_substep(Ctx &c, int rk, int bnd_end = 0, int bnd_begin = 0);
+hipError_t launch_substep(Ctx &c, int rk, int bnd_end = 0, int bnd_begin = 0, bool tick = false);
 constexpr int kNumPhases = 6;
 extern const char *const kPhaseNames[kNumPhases];
 hipError_t launch_phase(Ctx &c, int rk, int phase);

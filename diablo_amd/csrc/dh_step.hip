@@ -10,7 +10,8 @@
 //   k_rem_div_thomas
 //                 divergence, pressure-Poisson solve per (kx,kz), projection
 //                 and pressure update (channel.f:1103-1214, 1059-1065);
-//   k_courant_dt  the rest of COURANT (courant.f:45-62) on the device.
+//   k_courant_dt  the rest of COURANT (courant.f:45-62) on the device (in a
+//                 substep, a thread of the transform back).
 #include <type_traits>
 
 #include "dh_fft_dev.h"
@@ -1231,6 +1232,7 @@ struct FactorIn {
   double c1min[kMaxFields], c1max[kMaxFields];
   const double *dy, *dyf;
   int seg_rows;  // rows per register segment of the solve
+  int serial;    // 1: pivots by one thread in sequence (the mixed form)
 };
 
 // Row J (0..NY+1) of the system of field f: lower L, diagonal D, upper U,
@@ -1340,48 +1342,101 @@ __device__ __forceinline__ void cn_tables_body(const Clock *clk, const FactorIn 
     }
   }
   __syncthreads();
-  // the forward elimination is a recurrence: one thread, operands in LDS.
-  // Each row's operands are read one row ahead, so that their LDS latency
-  // overlaps the previous row's division instead of adding to it.
   double *tl = sm + 3 * nrow, *tb = sm + 4 * nrow, *tr = sm + 5 * nrow, *pf = sm + 6 * nrow, *pb = sm + 7 * nrow;
   const int sr = in.seg_rows;
-  if (threadIdx.x == 0) {
-    double bp = b[0], pfv = 0.0;
-    tl[0] = 0.0;
-    tb[0] = bp;
-    pf[0] = 0.0;
-    double an = a[1], bn = b[1], cn = c[0];
-    int js = (sr == 1) ? 0 : 1;  // J % sr
-    for (int J = 1; J < nrow; ++J) {
-      const double aj = an, bj = bn, cj = cn;
-      if (J + 1 < nrow) {
-        an = a[J + 1];
-        bn = b[J + 1];
-        cn = c[J];
+  // The forward elimination, B_J = D_J - L_J U_{J-1} / B_{J-1}, is a
+  // recurrence through a division.  One thread takes 0.19 us a row, and the
+  // tables outlast REM_DIV in the launch the two share (128 x 129 x 128: 34 us
+  // with one thread, 17.0 with the scan below, 16.9 without tables).  The rows of these systems have |D| = S + |L| + |U| with
+  // S >= 0 and -L D, -U D >= 0; then so has every pivot, |B_J| = s_J + |U_J|, and
+  //   s_J = S_J + |L_J| s_{J-1} / (s_{J-1} + |U_{J-1}|),
+  // a 2 x 2 matrix on s = n/d whose entries are not negative: products of such
+  // matrices don't cancel.  The first wave composes those of its lanes' rows by
+  // a scan, which gives each lane the pivot that its rows start from.  (The
+  // matrices of the recurrence as it stands cancel: 1e-8 in the pivots of stiff
+  // rows below a wall gradient.)  Rows of another form, and the mixed form, whose
+  // FP32 transforms carry a last-bit difference to 1e-7, keep the one thread.
+  const int lane = threadIdx.x;
+  if (lane < 64) {
+    const int R = (nrow + 63) / 64, r0 = lane * R, r1 = min(r0 + R, nrow);
+    double p00 = 1.0, p01 = 0.0, p10 = 0.0, p11 = 1.0;
+    auto rescale = [&] {  // by a power of two, which rounds nothing
+      int e;
+      (void)frexp(fmax(fmax(p00, p01), fmax(p10, p11)), &e);
+      p00 = ldexp(p00, -e);
+      p01 = ldexp(p01, -e);
+      p10 = ldexp(p10, -e);
+      p11 = ldexp(p11, -e);
+    };
+    bool ok = !in.serial;
+    for (int J = r0; J < r1 && ok; ++J) {
+      const double sg = copysign(1.0, b[J]), d = fabs(b[J]);
+      const double l = J > 0 ? -sg * a[J] : 0.0, u = -sg * c[J], up = J > 0 ? fabs(c[J - 1]) : 0.0;
+      const double x = d - l, sl = (x - u) + ((d - x) - l);  // the row's slack S, of its rounded entries
+      ok = l >= 0.0 && u >= 0.0 && sl >= 0.0;
+      const double m0 = sl + l, m1 = sl * up;
+      const double n0 = m0 * p00 + m1 * p10, n1 = m0 * p01 + m1 * p11;
+      p10 = p00 + up * p10;
+      p11 = p01 + up * p11;
+      p00 = n0;
+      p01 = n1;
+      rescale();
+    }
+    double bp = 0.0;
+    if (__all(ok)) {
+      for (int s = 1; s < 64; s *= 2) {
+        const double q00 = __shfl_up(p00, s), q01 = __shfl_up(p01, s);
+        const double q10 = __shfl_up(p10, s), q11 = __shfl_up(p11, s);
+        if (lane >= s) {
+          const double t00 = p00 * q00 + p01 * q10, t01 = p00 * q01 + p01 * q11;
+          const double t10 = p10 * q00 + p11 * q10, t11 = p10 * q01 + p11 * q11;
+          p00 = t00;
+          p01 = t01;
+          p10 = t10;
+          p11 = t11;
+          rescale();
+        }
       }
-      const double m = -aj / bp;
-      bp = bj + m * cj;
-      tl[J] = m;
-      tb[J] = bp;
-      pfv = (js == 0) ? m : pfv * m;
-      pf[J] = pfv;
-      js = (js + 1 == sr) ? 0 : js + 1;
+      bp = __shfl_up(p00 / p10, 1);  // s of the row below this lane's
+      if (lane > 0 && r0 < nrow) bp = copysign(bp + fabs(c[r0 - 1]), b[r0 - 1]);
+      for (int J = r0; J < r1; ++J) {
+        const double m = J > 0 ? -a[J] / bp : 0.0;
+        bp = J > 0 ? b[J] + m * c[J - 1] : b[0];
+        tl[J] = m;
+        tb[J] = bp;
+      }
+    } else if (lane == 0) {
+      bp = b[0];
+      tl[0] = 0.0;
+      tb[0] = bp;
+      double an = a[1], bn = b[1], cn = c[0];
+      for (int J = 1; J < nrow; ++J) {
+        const double aj = an, bj = bn, cj = cn;
+        if (J + 1 < nrow) {  // a row ahead, so that the reads' latency overlaps the division
+          an = a[J + 1];
+          bn = b[J + 1];
+          cn = c[J];
+        }
+        const double m = -aj / bp;
+        bp = bj + m * cj;
+        tl[J] = m;
+        tb[J] = bp;
+      }
     }
   }
   __syncthreads();
-  // the backward factors' quotients do not depend on one another: every
-  // thread takes some, and one thread chains the products
+  // the carry factors of a row: the products of its segment's multipliers up
+  // to it, and of the backward quotients from its segment's end down to it
   for (int J = threadIdx.x; J < nrow; J += blockDim.x) tr[J] = (tb[J] != 0.0) ? -c[J] / tb[J] : 0.0;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double pbv = 0.0;
-    int js = (nrow - 1) % sr;  // J % sr, counted down with J
-    for (int J = nrow - 1; J >= 0; --J) {
-      const double fj = tr[J];
-      pbv = (js == sr - 1 || J == nrow - 1) ? fj : fj * pbv;
-      pb[J] = pbv;
-      js = (js == 0) ? sr - 1 : js - 1;
-    }
+  for (int J = threadIdx.x; J < nrow; J += blockDim.x) {
+    const int s0 = J / sr * sr, s1 = min(s0 + sr, nrow) - 1;
+    double f = s0 ? tl[s0] : 0.0;
+    for (int i = s0 + 1; i <= J; ++i) f = f * tl[i];
+    pf[J] = f;
+    double g = tr[s1];
+    for (int i = s1 - 1; i >= J; --i) g = tr[i] * g;
+    pb[J] = g;
   }
   __syncthreads();
   const long long o = ((long long)rk * in.nfields + f) * nrow;
@@ -1606,41 +1661,12 @@ __global__ void __launch_bounds__(kSegThreads) k_solve_seg_b(const SolveArgs *__
   solve_seg_body<NS, P>(av[blockIdx.z]);
 }
 
-// COURANT (courant.f:45-62) from the CFL minimum of the solve kernel; the
-// solve tables for the new DELTA_T are rebuilt right after by k_cn_tables.
-__device__ __forceinline__ void courant_dt_body(Clock *clk, double dt_cap, int variable_dt, int update_dt) {
-  if (threadIdx.x != 0) return;
-  Clock &c = *clk;
-  // TEMP4 of this substep was fixed before COURANT (channel.f:80); the
-  // pressure update after REM_DIV (channel.f:1059-1065) still divides by it
-  c.h_cp = c.h_bar[2];
-  if (variable_dt && (c.time_step % update_dt) == 0) {
-    double dt = dt_cap;
-    const double m = __longlong_as_double((long long)c.cfl_min_bits);
-    if (m < dt) dt = m;
-    double DT;
-    if (dt <= 0)
-      DT = 0.0001;
-    else if (dt >= 999.)
-      DT = 999.0;
-    else
-      DT = dt;
-    c.dt = DT;
-    c.h_bar[0] = DT * (8.0 / 15.0);
-    c.h_bar[1] = DT * (2.0 / 15.0);
-    c.h_bar[2] = DT * (5.0 / 15.0);
-  }
-  c.cfl_min_bits = 0x7FF0000000000000ull;
+__global__ void k_courant_dt(CourantArgs a) {
+  if (threadIdx.x == 0) courant_dt_body(a.clk, a.dt_cap, a.variable_dt, a.update_dt);
 }
-struct CourantArgs {
-  Clock *clk;
-  double dt_cap;
-  int variable_dt, update_dt;
-};
-__global__ void k_courant_dt(CourantArgs a) { courant_dt_body(a.clk, a.dt_cap, a.variable_dt, a.update_dt); }
 __global__ void k_courant_dt_b(const CourantArgs *__restrict__ av) {
   const CourantArgs &a = av[blockIdx.z];
-  courant_dt_body(a.clk, a.dt_cap, a.variable_dt, a.update_dt);
+  if (threadIdx.x == 0) courant_dt_body(a.clk, a.dt_cap, a.variable_dt, a.update_dt);
 }
 
 // ---------------------------------------------------------------------------
@@ -2397,6 +2423,7 @@ static FactorIn make_factor_in(const Ctx &c) {
   in.dy = c.d_dy;
   in.dyf = c.d_dyf;
   in.seg_rows = c.fac.seg_rows;
+  in.serial = c.mixed ? 1 : 0;
   return in;
 }
 
@@ -3144,8 +3171,11 @@ static hipError_t launch_rem_div_cn(Ctx &c, int rk, int bnd_end, int bnd_begin) 
 // COURANT, then the solve tables for the new DELTA_T on the side stream: the
 // next solve is a substep away, so the rebuild runs beside this substep's
 // transform and pressure solve and is joined at the end of the substep.
+static CourantArgs courant_args(const Ctx &c) {
+  return CourantArgs{c.clock, c.dt_cap, c.p.variable_dt, c.p.update_dt};
+}
 static hipError_t launch_courant_dt(Ctx &c) {
-  const CourantArgs ca{c.clock, c.dt_cap, c.p.variable_dt, c.p.update_dt};
+  const CourantArgs ca = courant_args(c);
   return klaunch(c, (const void *)k_courant_dt, (const void *)k_courant_dt_b, dim3(1), dim3(64), 0, c.stream, ca);
 }
 static hipError_t launch_courant(Ctx &c) {
@@ -3195,7 +3225,8 @@ hipError_t join_side(Ctx &c) {
 // U2's solve and transform; the scalars' transform back, COURANT and
 // REM_DIV follow on the context stream once the branch has joined.  The
 // kernels and their arithmetic are those of launch_phase.
-hipError_t launch_substep(Ctx &c, int rk, int bnd_end, int bnd_begin) {
+// tick: the substep opens a step (TIME_STEP += 1, diablo.f:66).
+hipError_t launch_substep(Ctx &c, int rk, int bnd_end, int bnd_begin, bool tick) {
   const int courant = (c.p.variable_dt && rk == 2) ? 1 : 0;
   // after COURANT the CN tables of the new DELTA_T are built in REM_DIV's
   // launch (a fork to a side stream and its join cost more on the device
@@ -3205,13 +3236,17 @@ hipError_t launch_substep(Ctx &c, int rk, int bnd_end, int bnd_begin) {
   hipError_t e;
 #define SCHK(expr) \
   if ((e = (expr)) != hipSuccess) return e;
+  // the step's opening goes with its first launch, except with LES, whose
+  // first launch reads TIME_STEP
+  const bool own_tick = tick && (c.les || c.recording);
+  if (own_tick) SCHK(launch_step_boundary(c, false, true));
   if (c.les) {
     // les_chan's BCs and the model's strain in one launch, then its inverse
     // transforms and U's in one launch (both read the BC'd Fourier copy)
     SCHK(launch_les_strain_and_state(c, c.stream));
     SCHK(launch_les_model_rest(c, c.stream));
   } else {
-    SCHK(launch_state_to_phys(c));
+    SCHK(launch_state_to_phys(c, tick && !own_tick));
   }
   if (flat_substep(c)) {
     // one launch per phase, in launch_phase's order (the solve tables of a
@@ -3219,8 +3254,11 @@ hipError_t launch_substep(Ctx &c, int rk, int bnd_end, int bnd_begin) {
     SCHK(launch_nonlinear_range(c, rk, 0, c.nfields, c.stream));
     SCHK(c.les ? launch_solve_les_range(c, rk, courant, 0, c.nfields, c.stream)
                : launch_solve_range(c, rk, courant, 0, c.nfields, c.stream));
-    if (courant) SCHK(fuse_tables ? launch_courant_dt(c) : launch_courant(c));
-    SCHK(launch_step_to_four(c, 0, c.nfields, c.stream));
+    // COURANT's new DELTA_T by one thread of the transform back, which reads
+    // nothing of the clock
+    const CourantArgs ca = courant_args(c);
+    if (courant && !fuse_tables) SCHK(launch_courant(c));
+    SCHK(launch_step_to_four(c, 0, c.nfields, c.stream, fuse_tables ? &ca : nullptr));
     SCHK(fuse_tables ? launch_rem_div_cn(c, rk, bnd_end, bnd_begin) : launch_rem_div(c, rk, bnd_end, bnd_begin));
     return join_side(c);
   }
