@@ -175,6 +175,18 @@ double dt_cap_of(const Ctx &c) {
   return dt;
 }
 
+// Segments of a column in the solve of the context's form.  FP64: kColSegs of
+// up to kColRows rows (k_solve_cols); mixed: 4 or 8 of up to kSegRows
+// (k_solve_seg).
+static void set_solve_segments(Ctx &c) {
+  const int nrow = c.g.ny + 2;
+  if (c.mixed)
+    c.fac.nseg = (nrow <= 4 * kSegRows) ? 4 : 8;
+  else
+    c.fac.nseg = kColSegs;
+  c.fac.seg_rows = (nrow + c.fac.nseg - 1) / c.fac.nseg;
+}
+
 int rebuild_tables(Ctx &c) {
   HIPCHK(launch_cn_tables(c, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
@@ -239,6 +251,7 @@ int dh_create(const dh_params *p, dh_ctx **out) {
   c.gp = c.lds_bytes > kLdsMax;
   if (c.gp && gp_stage_elems(g) < std::max(g.ls, 2 * g.nz))
     return reject("x-z plane too large (a row or a column of it does not fit the staging buffer)");
+  static_assert(8 * kSegRows == kColSegs * kColRows, "both forms take the same NY");
   if (g.ny + 2 > 8 * kSegRows) return reject("NY+2 is beyond the column solver's register segments (8 x 36 rows)");
   int thr = (g.nz * g.lw + 7) / 8;
   thr = ((thr + 63) / 64) * 64;
@@ -346,8 +359,7 @@ int dh_create(const dh_params *p, dh_ctx **out) {
   ACHK(dalloc(&c.fac.tb, 3 * (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.tc, 3 * (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.tr, 3 * (size_t)c.nfields * nyy));
-  c.fac.nseg = (nyy <= 4 * (size_t)kSegRows) ? 4 : 8;
-  c.fac.seg_rows = (int)((nyy + c.fac.nseg - 1) / c.fac.nseg);
+  set_solve_segments(c);
   ACHK(dalloc(&c.fac.isbc, (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.vconst, (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.bcl, (size_t)c.nfields * nyy));
@@ -694,7 +706,9 @@ int dh_set_mixed_precision(dh_ctx *h, int32_t on) {
   }
   c.mixed = (on != 0);
   drop_graphs(c);  // the captured steps launch the other form's kernels
-  return DH_OK;
+  set_solve_segments(c);
+  // the solve tables are laid out by segments, and each form has its pivots
+  return c.grid_set ? rebuild_tables(c) : DH_OK;
 }
 
 int dh_mixed_precision(dh_ctx *h) { return h ? (h->c.mixed ? 1 : 0) : DH_EARG; }

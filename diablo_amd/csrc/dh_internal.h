@@ -71,9 +71,11 @@ struct Clock {
 // Parallel-cyclic-reduction tables of the y-implicit (Crank-Nicolson)
 // matrices, one set per RK substep and field; with LES off each matrix
 // depends only on j, so every (x,z) column of a field shares it.
-// Rows of one column held by one lane of the Crank-Nicolson solve; a column
-// is split into 4 (NY+2 <= 144) or 8 such segments.
+// Most rows of one column held by one lane of the mixed form's Crank-Nicolson
+// solve; a column is split into 4 (NY+2 <= 144) or 8 such segments.
 constexpr int kSegRows = 36;
+// The FP64 form's solve takes 16 segments of up to 18 rows.
+constexpr int kColSegs = 16, kColRows = 18;
 constexpr int kStepsPerGraph = 8;  // time steps captured in one graph for long runs
 // Most rows 2..NY of one (kx,kz) mode's pressure-Poisson sweep that a thread
 // of REM_DIV holds in registers (23 of them per row).
@@ -113,7 +115,7 @@ struct RealFactors {
   double *vconst;             // [field][row]
   double *bcl, *bcd, *bcu;    // [field][row] coefficients of the boundary rows (isbc = 1)
   int seg_rows;               // rows per register segment of a column
-  int nseg;                   // segments per column (4 or 8)
+  int nseg;                   // segments per column
 };
 
 // A launch, event record or stream wait of the step sequence, as the

@@ -4,7 +4,8 @@
 //                 their forward transforms, RK combination, explicit half of
 //                 the y-viscous term and the inverse transform of the
 //                 right-hand side (channel.f:77-626);
-//   k_solve_seg   real tridiagonal Crank-Nicolson solve of every (x,z)
+//   k_solve_cols, k_solve_seg (mixed form)
+//                 real tridiagonal Crank-Nicolson solve of every (x,z)
 //                 column, and the CFL minimum (channel.f:771-1029,
 //                 courant.f:34-43);
 //   k_rem_div_thomas
@@ -1473,6 +1474,7 @@ __global__ void __launch_bounds__(256) k_cn_tables_b(const CnArgs *__restrict__ 
 //   backward: each segment sweeps from a zero carry, y_J = (g_J - TC_J
 //             y_{J+1}) / TB_J (quotient from 1/TB_J, the same double as the
 //             division); the carries x_b pass down, and x_J = y_J + PB_J x_b.
+// (k_solve_cols: through LDS.)
 // The first segment's forward values and the last segment's backward values
 // are the reference's own; the others differ from a single sweep by the
 // rounding of the carry terms.
@@ -1496,14 +1498,14 @@ struct SolveArgs {
 
 constexpr int kSegThreads = 256;
 
-template <int NS, class P>
+// The mixed form's solve: FP32 rows, FP64 arithmetic.
+template <int NS>
 __device__ __forceinline__ void solve_seg_body(const SolveArgs &a) {
 #pragma clang fp contract(off)
   constexpr int CW = 64 / NS;  // columns per wave
   constexpr int SR = kSegRows;
   // tables in LDS, padded to NS * seg_rows rows
-  __shared__ double TL[NS * SR], TB[NS * SR], TC[NS * SR], TR[NS * SR], PF[NS * SR], PB[NS * SR], VC[NS * SR];
-  __shared__ int IB[NS * SR];
+  __shared__ double TL[NS * SR], TB[NS * SR], TC[NS * SR], TR[NS * SR], PF[NS * SR], PB[NS * SR];
   __shared__ double red[kSegThreads / 64];
   const Geo &g = a.g;
   const int f = a.f0 + blockIdx.y;
@@ -1519,8 +1521,6 @@ __device__ __forceinline__ void solve_seg_body(const SolveArgs &a) {
     TR[i] = in ? a.fac.tr[to + i] : 1.0;
     PF[i] = in ? a.fac.pf[to + i] : 0.0;
     PB[i] = in ? a.fac.pb[to + i] : 0.0;
-    VC[i] = in ? a.fac.vconst[(long long)f * nrow + i] : 0.0;
-    IB[i] = in ? a.fac.isbc[(long long)f * nrow + i] : 1;
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1531,31 +1531,22 @@ __device__ __forceinline__ void solve_seg_body(const SolveArgs &a) {
   const int nr = min(sr, max(nrow - r0, 0));
   // rows are addressed from the field's (uniform) base with 32-bit element
   // offsets i pp + col (a field is below 2^31 elements)
-  P *const Ub = static_cast<P *>(a.dst[f]);
-  const P *const Rb = static_cast<const P *>(a.rphys) + (long long)f * a.fs;
+  float *const Ub = static_cast<float *>(a.dst[f]);
+  const float *const Rb = static_cast<const float *>(a.rphys) + (long long)f * a.fs;
   const unsigned ppu = (unsigned)pp, colu = (unsigned)col;
   auto ro_ = [&](int i) { return (unsigned)i * ppu + colu; };
   // the mixed form solves for the increment d = U_new - U_old: every row's
   // right-hand side is in R (interior rows from the nonlinear pass,
   // boundary rows from k_bc_increment)
-  constexpr bool DELTA = sizeof(P) == sizeof(float);
-  P *const Uob = DELTA ? static_cast<P *>(a.uold) + (long long)f * a.fs : nullptr;
-  // right-hand sides: the boundary constant or R
+  float *const Uob = static_cast<float *>(a.uold) + (long long)f * a.fs;
   double v[SR];
 #pragma unroll
   for (int q = 0; q < SR; ++q) {
     const int i = r0 + q;
-    v[q] = (live && q < nr && (DELTA || !IB[i])) ? Rb[ro_(i)] : 0.0;
+    v[q] = (live && q < nr) ? Rb[ro_(i)] : 0.0;
     // FP32 rows are converted in chunks, so that the loads in flight and
     // their FP64 values do not both hold all rows' registers
-    if (DELTA && q % 12 == 11) __builtin_amdgcn_sched_barrier(0);
-  }
-  if constexpr (!DELTA) {
-#pragma unroll
-    for (int q = 0; q < SR; ++q) {
-      const int i = r0 + q;
-      if (q < nr && IB[i]) v[q] = VC[i];
-    }
+    if (q % 12 == 11) __builtin_amdgcn_sched_barrier(0);
   }
   // forward sweep within the segment from a zero carry
   double hp = 0.0, hend = 0.0;
@@ -1612,31 +1603,23 @@ __device__ __forceinline__ void solve_seg_body(const SolveArgs &a) {
   for (int q = 0; q < SR; ++q) {
     const int i = r0 + q;
     const double x = (seg == NS - 1) ? v[q] : v[q] + PB[i] * xin;
-    if (live && q < nr && i >= wlo && i <= whi) {
-      Ub[ro_(i)] = x;
-      if (!DELTA && cour && i >= 1 && i <= NY) {
-        const double dl = (f == 1) ? g.dy[i] : dxf;
-        dtmin = fmin(dtmin, a.cfl * dl / fabs(x));
-      }
-    }
+    if (live && q < nr && i >= wlo && i <= whi) Ub[ro_(i)] = x;
   }
   // the mixed form: the new values U_old + d, for COURANT and for the
   // physical field of a scalar (which persists); in a loop of its own that
   // reads d back from U (this lane's own stores), so that the rows' values
   // need not stay in registers
-  if constexpr (DELTA) {
-    if (cour || f >= 3) {
+  if (cour || f >= 3) {
 #pragma unroll 6
-      for (int q = 0; q < SR; ++q) {
-        const int i = r0 + q;
-        if (live && q < nr && i >= wlo && i <= whi) {
-          const double x = (double)Ub[ro_(i)];
-          const double un = (a.four[f][(long long)i * g.pf].x + (double)Uob[ro_(i)]) + x;
-          if (f >= 3) Uob[ro_(i)] = (P)un;
-          if (cour && i >= 1 && i <= NY) {
-            const double dl = (f == 1) ? g.dy[i] : dxf;
-            dtmin = fmin(dtmin, a.cfl * dl / fabs(un));
-          }
+    for (int q = 0; q < SR; ++q) {
+      const int i = r0 + q;
+      if (live && q < nr && i >= wlo && i <= whi) {
+        const double x = (double)Ub[ro_(i)];
+        const double un = (a.four[f][(long long)i * g.pf].x + (double)Uob[ro_(i)]) + x;
+        if (f >= 3) Uob[ro_(i)] = (float)un;
+        if (cour && i >= 1 && i <= NY) {
+          const double dl = (f == 1) ? g.dy[i] : dxf;
+          dtmin = fmin(dtmin, a.cfl * dl / fabs(un));
         }
       }
     }
@@ -1652,13 +1635,133 @@ __device__ __forceinline__ void solve_seg_body(const SolveArgs &a) {
     }
   }
 }
-template <int NS, class P>
-__global__ void __launch_bounds__(kSegThreads) k_solve_seg(SolveArgs a) {
-  solve_seg_body<NS, P>(a);
+
+constexpr int kColCols = 32;  // columns per block
+
+// The FP64 solve: a block takes 32 neighbouring columns in 16 segments of up to
+// SR rows, one thread per segment and column (columns fastest, so that a wave's
+// loads and stores are whole 256-byte pieces of two rows), and the carries cross
+// the segments through LDS.  It is bound by memory for many columns and by
+// the chain of rows for few, so rows stay few per thread: with a column in 4 or
+// 8 lanes of 36 rows it took 174 us at 256 x 193 x 256 (1.2 GB; 127 in this form),
+// 26 at 128 x 129 x 128 (25), 19.7 at 256 x 257 x 4 (11.9) and 13.6 at
+// 64 x 65 x 4 (5.3).  32 segments take 10.4, but 199 at 256 x 193 x 256; 16
+// columns a block 139 there, 64 columns 145.
+template <int SR>
+__device__ __forceinline__ void solve_cols_body(const SolveArgs &a) {
+#pragma clang fp contract(off)
+  constexpr int NSEG = kColSegs, CB = kColCols, NR = NSEG * SR, NT = NSEG * CB;
+  __shared__ double TL[NR], TB[NR], TC[NR], TR[NR], PF[NR], PB[NR], VC[NR];
+  __shared__ int IB[NR];
+  __shared__ double H[NSEG * CB];
+  __shared__ double red[NT / 64];
+  const Geo &g = a.g;
+  const int f = a.f0 + blockIdx.y;
+  const int NY = g.ny, nrow = NY + 2;
+  const int sr = a.fac.seg_rows;
+  const int cl = threadIdx.x & (CB - 1), seg = threadIdx.x / CB;
+  const unsigned ppu = (unsigned)g.pp, col = blockIdx.x * CB + cl;
+  const bool live = col < ppu;
+  const unsigned colu = min(col, ppu - 1);
+  const int r0 = seg * sr, nr = min(sr, max(nrow - r0, 0));
+  double *const Ub = static_cast<double *>(a.dst[f]);
+  const double *const Rb = static_cast<const double *>(a.rphys) + (long long)f * a.fs;
+  auto ro_ = [&](int i) { return (unsigned)i * ppu + colu; };
+  // the rows first: their latency passes beside the tables'
+  double v[SR];
+#pragma unroll
+  for (int q = 0; q < SR; ++q) v[q] = Rb[ro_(min(r0 + q, nrow - 1))];
+  // rows beyond a segment's: the forward carry passes through them (TL = 1),
+  // the backward sweep starts from zero in them
+  const long long to = ((long long)a.rk * a.nfields + f) * nrow, fo = (long long)f * nrow;
+  for (int e = threadIdx.x; e < NR; e += NT) {
+    const int s = e / SR, q = e - s * SR, i = s * sr + q;
+    const bool in = q < sr && i < nrow;
+    TL[e] = in ? a.fac.tl[to + i] : 1.0;
+    TB[e] = in ? a.fac.tb[to + i] : 1.0;
+    TC[e] = in ? a.fac.tc[to + i] : 0.0;
+    TR[e] = in ? a.fac.tr[to + i] : 1.0;
+    PF[e] = in ? a.fac.pf[to + i] : 0.0;
+    PB[e] = in ? a.fac.pb[to + i] : 0.0;
+    VC[e] = in ? a.fac.vconst[fo + i] : 0.0;
+    IB[e] = in ? a.fac.isbc[fo + i] : 1;
+  }
+  __syncthreads();
+  const int t0 = seg * SR;
+  // right-hand sides (the boundary constant or R), forward from a zero carry
+  double hp = 0.0;
+#pragma unroll
+  for (int q = 0; q < SR; ++q) {
+    const double d = IB[t0 + q] ? VC[t0 + q] : v[q];
+    hp = d + TL[t0 + q] * hp;
+    v[q] = hp;
+  }
+  H[threadIdx.x] = hp;
+  __syncthreads();
+  // g_in(s) = g_end(s-1), g_end = h_end + PF_end g_in
+  double gin = 0.0;
+  for (int s = 0; s < seg; ++s) gin = H[s * CB + cl] + PF[s * SR + sr - 1] * gin;
+#pragma unroll
+  for (int q = 0; q < SR; ++q) v[q] = (seg == 0) ? v[q] : v[q] + PF[t0 + q] * gin;
+  // backward from a zero carry
+  double yn = 0.0;
+#pragma unroll
+  for (int q = SR - 1; q >= 0; --q) {
+    const double b = TB[t0 + q];
+    const double y = (b != 0.0) ? div_by_recip(v[q] - TC[t0 + q] * yn, b, TR[t0 + q]) : 0.0;
+    v[q] = y;
+    yn = (q < nr) ? y : 0.0;
+  }
+  __syncthreads();
+  H[threadIdx.x] = (nr > 0) ? yn : 0.0;
+  __syncthreads();
+  // x_in(s) = x_start(s+1), x_start = y_start + PB_start x_in
+  double xin = 0.0;
+  for (int s = NSEG - 1; s > seg; --s) xin = H[s * CB + cl] + PB[s * SR] * xin;
+  const bool cour = a.courant && f < 3;
+  const double dxf = (f == 0) ? a.dx : a.dz;
+  double dtmin = __longlong_as_double(0x7FF0000000000000ll);
+  const int wlo = a.wlo[f], whi = a.whi[f];
+#pragma unroll
+  for (int q = 0; q < SR; ++q) {
+    const int i = r0 + q;
+    const double x = (r0 + sr >= nrow) ? v[q] : v[q] + PB[t0 + q] * xin;
+    if (live && q < nr && i >= wlo && i <= whi) {
+      Ub[ro_(i)] = x;
+      if (cour && i >= 1 && i <= NY) {
+        const double dl = (f == 1) ? g.dy[i] : dxf;
+        dtmin = fmin(dtmin, a.cfl * dl / fabs(x));
+      }
+    }
+  }
+  if (cour) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int o = 32; o > 0; o >>= 1) dtmin = fmin(dtmin, __shfl_down(dtmin, o));
+    if (lane == 0) red[w] = dtmin;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double m = red[0];
+      for (int q = 1; q < NT / 64; ++q) m = fmin(m, red[q]);
+      if (m >= 0.0) atomicMin(&a.clk->cfl_min_bits, (unsigned long long)__double_as_longlong(m));
+    }
+  }
 }
-template <int NS, class P>
+template <int SR>
+__global__ void __launch_bounds__(kColSegs * kColCols) k_solve_cols(SolveArgs a) {
+  solve_cols_body<SR>(a);
+}
+template <int SR>
+__global__ void __launch_bounds__(kColSegs * kColCols) k_solve_cols_b(const SolveArgs *__restrict__ av) {
+  solve_cols_body<SR>(av[blockIdx.z]);
+}
+
+template <int NS>
+__global__ void __launch_bounds__(kSegThreads) k_solve_seg(SolveArgs a) {
+  solve_seg_body<NS>(a);
+}
+template <int NS>
 __global__ void __launch_bounds__(kSegThreads) k_solve_seg_b(const SolveArgs *__restrict__ av) {
-  solve_seg_body<NS, P>(av[blockIdx.z]);
+  solve_seg_body<NS>(av[blockIdx.z]);
 }
 
 __global__ void k_courant_dt(CourantArgs a) {
@@ -2644,16 +2747,22 @@ static hipError_t launch_solve_range(Ctx &c, int rk, int courant, int f0, int f1
                            dim3((unsigned)((c.g.pp + 255) / 256), f1 - f0), dim3(256), 0, st, a);
     if (e != hipSuccess) return e;
     if (c.fac.nseg == 4)
-      return klaunch(c, (const void *)k_solve_seg<4, float>, (const void *)k_solve_seg_b<4, float>, grid,
+      return klaunch(c, (const void *)k_solve_seg<4>, (const void *)k_solve_seg_b<4>, grid,
                      dim3(kSegThreads), 0, st, a);
-    return klaunch(c, (const void *)k_solve_seg<8, float>, (const void *)k_solve_seg_b<8, float>, grid,
+    return klaunch(c, (const void *)k_solve_seg<8>, (const void *)k_solve_seg_b<8>, grid,
                    dim3(kSegThreads), 0, st, a);
   }
-  if (c.fac.nseg == 4)
-    return klaunch(c, (const void *)k_solve_seg<4, double>, (const void *)k_solve_seg_b<4, double>, grid,
-                   dim3(kSegThreads), 0, st, a);
-  return klaunch(c, (const void *)k_solve_seg<8, double>, (const void *)k_solve_seg_b<8, double>, grid,
-                 dim3(kSegThreads), 0, st, a);
+  auto cols_launch = [&](auto rows) {
+    constexpr int SR = decltype(rows)::value;
+    return klaunch(c, (const void *)k_solve_cols<SR>, (const void *)k_solve_cols_b<SR>,
+                   dim3((unsigned)((c.g.pp + kColCols - 1) / kColCols), f1 - f0), dim3(kColSegs * kColCols), 0, st, a);
+  };
+  using std::integral_constant;
+  const int sr = c.fac.seg_rows;
+  if (sr <= 5) return cols_launch(integral_constant<int, 5>{});
+  if (sr <= 9) return cols_launch(integral_constant<int, 9>{});
+  if (sr <= 13) return cols_launch(integral_constant<int, 13>{});
+  return cols_launch(integral_constant<int, kColRows>{});
 }
 
 static hipError_t launch_solve(Ctx &c, int rk, int courant) {
