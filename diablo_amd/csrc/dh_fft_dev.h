@@ -721,8 +721,12 @@ __device__ void rows_inv_reg64(C *A, const Geo &g, const TablesT<C> &T, Store st
 // (FFT_XZ_TO_FOURIER's r2c, mpi.f:1490-1506).  With m = t + 4r (r < 8) and
 // k = k1 + 8 k2 (k1 < 8, k2 < 4):
 //   Z_{k1+8k2} = sum_t W4^{t k2} W32^{t k1} sum_r W8^{r k1} x_{t+4r}.
-template <class C, class Load>
-__device__ void rows_fwd_reg32(C *A, const Geo &g, const TablesT<C> &T, Load load) {
+// Samples come from eval(fetch(z, m)), the fetches of a group ahead of its
+// arithmetic, and MERGE adds another product's transform, both as in
+// rows_fwd_reg64.
+template <bool MERGE = false, class C, class Fetch, class Eval>
+__device__ void rows_fwd_reg32(C *A, const Geo &g, const TablesT<C> &T, Fetch fetch, Eval eval,
+                               const double *kxv = nullptr) {
   using S = Sc<C>;
   const int lane = threadIdx.x & 63, rho = lane >> 2, t = lane & 3;
   const int nw = blockDim.x >> 6;
@@ -730,9 +734,23 @@ __device__ void rows_fwd_reg32(C *A, const Geo &g, const TablesT<C> &T, Load loa
   for (int slab = threadIdx.x >> 6; slab * 16 < g.nz; slab += nw) {
     const int z = slab * 16 + rho;  // < NZ: these rows require NZ % 16 == 0
     C *row = A + z * g.ls;
+    using Raw = decltype(fetch(0, 0));
+    constexpr int G = sizeof(Raw) > 48 ? 4 : 8;
     C v[8];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] = load(z, t + 4 * r);
+    for (int r0 = 0; r0 < 8; r0 += G) {
+      Raw raw[G];
+#pragma unroll
+      for (int r = 0; r < G; ++r) raw[r] = fetch(z, t + 4 * (r0 + r));
+      if constexpr (sizeof(Raw) > sizeof(C)) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < G; ++r) v[r0 + r] = eval(raw[r]);
+    }
+    C prev[MERGE ? 8 : 1];  // the other product's outputs of this lane
+    if constexpr (MERGE) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) prev[i] = row[min(2 * t + i / 4 + 8 * (i & 3), g.nkx)];
+    }
     dft_small<8, false>(v);  // v[k1] = sum_r W8^{r k1} x_{t+4r}
 #pragma unroll
     for (int k1 = 1; k1 < 8; ++k1) v[k1] = cmul(v[k1], T.twr[t * k1]);  // W32^{t k1}
@@ -771,10 +789,20 @@ __device__ void rows_fwd_reg32(C *A, const Geo &g, const TablesT<C> &T, Load loa
         C a = mkc<C>(S(0.5) * (zk.x + zmk.x), S(0.5) * (zk.y - zmk.y));
         C b = mkc<C>(S(0.5) * (zk.x - zmk.x), S(0.5) * (zk.y + zmk.y));
         C wb = cmul(T.twx[k], b);
-        if (k <= g.nkx) row[k] = mkc<C>(div_by_recip(a.x + wb.y, nxd, rnx), div_by_recip(a.y - wb.x, nxd, rnx));
+        C x = mkc<C>(div_by_recip(a.x + wb.y, nxd, rnx), div_by_recip(a.y - wb.x, nxd, rnx));
+        if constexpr (MERGE) {
+          const C ik = cmul_ik(S(kxv[min(k, g.nkx)]), prev[4 * h + k2]);
+          x = mkc<C>(ik.x + x.x, ik.y + x.y);
+        }
+        if (k <= g.nkx) row[k] = x;
       }
   }
   lds_barrier();
+}
+
+template <class C, class Load>
+__device__ __forceinline__ void rows_fwd_reg32(C *A, const Geo &g, const TablesT<C> &T, Load load) {
+  rows_fwd_reg32<false>(A, g, T, load, [](C v) { return v; });
 }
 
 // Inverse x transform of every row for NX = 64 (FFT_XZ_TO_PHYSICAL's c2r,

@@ -431,11 +431,14 @@ __device__ __forceinline__ void nonlinear_pass(const StepArgs &a, C *A) {
     lds_barrier();
   };
   const int pz = (c == 0) ? 0 : 1;  // the ikz product; the other of 0, 1 takes ikx
-  if constexpr (REG) {
-    // x transforms in registers.  The ikz product has its own z transform;
-    // the ikx product and the plain y-flux product (p = 2) share one: the
-    // x-transformed ikx product is scaled by i KX and added to the y flux's
-    // (both transforms are linear and KX is constant along z).
+  // x transforms in registers (X64: NX = 128, else NX = 64).  The ikz product
+  // has its own z transform; the ikx product and the plain y-flux product (p =
+  // 2) share one: the x-transformed ikx product is scaled by i KX and added to
+  // the y flux's (both transforms are linear and KX is constant along z).
+  // NX = 64 in this form (LES at 64 x 97 x 64): 38.9 us, where one product after
+  // the other, each sample's form decided as it is loaded, took 46.8.
+  auto products = [&](auto x64) {
+    constexpr bool X64 = decltype(x64)::value;
     auto rows = [&](int p, auto merge) {
       constexpr bool MERGE = decltype(merge)::value;
       const Prod<C> pr = make_prod<C>(a, c, p, J);
@@ -443,9 +446,12 @@ __device__ __forceinline__ void nonlinear_pass(const StepArgs &a, C *A) {
       // straight-line code ahead of the arithmetic
       auto run = [&](auto K) {
         constexpr int KIND = decltype(K)::value;
-        rows_fwd_reg64<MERGE>(
-            A, g, T, [&](int z, int xp) { return fetch_prod<KIND, C>(pr, (long long)z * g.nx + 2 * xp); },
-            [&](const ProdRaw<KIND, C> &r) { return eval_raw<KIND, C>(pr, r); }, g.kx);
+        auto fetch = [&](int z, int xp) { return fetch_prod<KIND, C>(pr, (long long)z * g.nx + 2 * xp); };
+        auto eval = [&](const ProdRaw<KIND, C> &r) { return eval_raw<KIND, C>(pr, r); };
+        if constexpr (X64)
+          rows_fwd_reg64<MERGE>(A, g, T, fetch, eval, g.kx);
+        else
+          rows_fwd_reg32<MERGE>(A, g, T, fetch, eval, g.kx);
       };
       // forms: the y fluxes (p = 2) are 2 or 4, the others 0, 1 or 3
       if constexpr (MERGE) {
@@ -464,22 +470,30 @@ __device__ __forceinline__ void nonlinear_pass(const StepArgs &a, C *A) {
     rows(2, std::true_type{});
     plane_cols_fwd(A, g, T);
     accumulate(2);
-  } else {
+  };
+  // the LDS rows: one product after the other
+  auto products_lds = [&] {
     for (int p = 0; p < 3; ++p) {
       const Prod<C> pr = make_prod<C>(a, c, p, J);
-      if (R32 && a.rows32) {
-        rows_fwd_reg32(A, g, T, [&](int z, int xp) { return eval_prod(pr, (long long)z * g.nx + 2 * xp); });
-      } else {
-        for (int t0 = threadIdx.x >> 6; t0 < lt.ntiles; t0 += nw) {
-          int z, xp;
-          if (lt.at(g, t0, z, xp)) A[phys_slot(T, g, z, xp)] = eval_prod(pr, (long long)z * g.nx + 2 * xp);
-        }
-        lds_barrier();
-        plane_rows_fwd(A, g, T);
+      for (int t0 = threadIdx.x >> 6; t0 < lt.ntiles; t0 += nw) {
+        int z, xp;
+        if (lt.at(g, t0, z, xp)) A[phys_slot(T, g, z, xp)] = eval_prod(pr, (long long)z * g.nx + 2 * xp);
       }
+      lds_barrier();
+      plane_rows_fwd(A, g, T);
       plane_cols_fwd(A, g, T);
       accumulate(p == 2 ? 2 : (p == pz ? 0 : 1));
     }
+  };
+  if constexpr (REG) {
+    products(std::true_type{});
+  } else if constexpr (R32) {
+    if (a.rows32)
+      products(std::false_type{});
+    else
+      products_lds();
+  } else {
+    products_lds();
   }
   // RK combination (channel.f:88-167, 581-595; scalars 254-270, 723-729),
   // new CF stored, CR scattered into LDS for the inverse transform.
@@ -2739,10 +2753,9 @@ static hipError_t launch_solve_range(Ctx &c, int rk, int courant, int f0, int f1
   a.cfl = c.p.cfl;
   a.dx = c.p.lx / c.g.nx;
   a.dz = c.p.lz / c.g.nz;
-  const int cols = (kSegThreads / 64) * (64 / c.fac.nseg);  // columns per block
-  const int nb = (int)((c.g.pp + cols - 1) / cols);
-  const dim3 grid(nb, f1 - f0);
   if (c.mixed) {
+    const int cols = (kSegThreads / 64) * (64 / c.fac.nseg);  // columns per block
+    const dim3 grid((unsigned)((c.g.pp + cols - 1) / cols), f1 - f0);
     hipError_t e = klaunch(c, (const void *)k_bc_increment, (const void *)k_bc_increment_b,
                            dim3((unsigned)((c.g.pp + 255) / 256), f1 - f0), dim3(256), 0, st, a);
     if (e != hipSuccess) return e;
