@@ -1510,6 +1510,14 @@ struct SolveArgs {
   double cfl, dx, dz;
 };
 
+// COURANT's minimum, one thread per block: only a block below what it reads of
+// the minimum so far (which only falls) goes to the atomic, which all blocks
+// queue at.
+__device__ __forceinline__ void cfl_min(Clock *clk, double m) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(m);
+  if (m >= 0.0 && b < *(volatile unsigned long long *)&clk->cfl_min_bits) atomicMin(&clk->cfl_min_bits, b);
+}
+
 constexpr int kSegThreads = 256;
 
 // The mixed form's solve: FP32 rows, FP64 arithmetic.
@@ -1645,7 +1653,7 @@ __device__ __forceinline__ void solve_seg_body(const SolveArgs &a) {
     if (threadIdx.x == 0) {
       double m = red[0];
       for (int q = 1; q < (int)(blockDim.x >> 6); ++q) m = fmin(m, red[q]);
-      if (m >= 0.0) atomicMin(&a.clk->cfl_min_bits, (unsigned long long)__double_as_longlong(m));
+      cfl_min(a.clk, m);
     }
   }
 }
@@ -1734,7 +1742,7 @@ __device__ __forceinline__ void solve_cols_body(const SolveArgs &a) {
   for (int s = NSEG - 1; s > seg; --s) xin = H[s * CB + cl] + PB[s * SR] * xin;
   const bool cour = a.courant && f < 3;
   const double dxf = (f == 0) ? a.dx : a.dz;
-  double dtmin = __longlong_as_double(0x7FF0000000000000ll);
+  double dtmin = __longlong_as_double(0x7FF0000000000000ll), xmax = 0.0;
   const int wlo = a.wlo[f], whi = a.whi[f];
 #pragma unroll
   for (int q = 0; q < SR; ++q) {
@@ -1743,11 +1751,16 @@ __device__ __forceinline__ void solve_cols_body(const SolveArgs &a) {
     if (live && q < nr && i >= wlo && i <= whi) {
       Ub[ro_(i)] = x;
       if (cour && i >= 1 && i <= NY) {
-        const double dl = (f == 1) ? g.dy[i] : dxf;
-        dtmin = fmin(dtmin, a.cfl * dl / fabs(x));
+        if (f == 1)
+          dtmin = fmin(dtmin, a.cfl * g.dy[i] / fabs(x));
+        else
+          xmax = fmax(xmax, fabs(x));
       }
     }
   }
+  // one spacing: the least quotient is that of the largest velocity, to the bit
+  // (rounding keeps the order)
+  if (cour && f != 1) dtmin = a.cfl * dxf / xmax;
   if (cour) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int o = 32; o > 0; o >>= 1) dtmin = fmin(dtmin, __shfl_down(dtmin, o));
@@ -1756,7 +1769,7 @@ __device__ __forceinline__ void solve_cols_body(const SolveArgs &a) {
     if (threadIdx.x == 0) {
       double m = red[0];
       for (int q = 1; q < NT / 64; ++q) m = fmin(m, red[q]);
-      if (m >= 0.0) atomicMin(&a.clk->cfl_min_bits, (unsigned long long)__double_as_longlong(m));
+      cfl_min(a.clk, m);
     }
   }
 }
@@ -2966,7 +2979,7 @@ __global__ void __launch_bounds__(kLesSolveThreads) k_solve_les(LesSolveArgs a) 
     if (threadIdx.x == 0) {
       double m = red[0];
       for (int q = 1; q < (int)(blockDim.x >> 6); ++q) m = fmin(m, red[q]);
-      if (m >= 0.0) atomicMin(&a.clk->cfl_min_bits, (unsigned long long)__double_as_longlong(m));
+      cfl_min(a.clk, m);
     }
   }
 }
@@ -3178,7 +3191,7 @@ __global__ void __launch_bounds__(kLesPartThreads) k_solve_les_part(LesSolveArgs
     if (threadIdx.x == 0) {
       double m = red[0];
       for (int q = 1; q < (int)(blockDim.x >> 6); ++q) m = fmin(m, red[q]);
-      if (m >= 0.0) atomicMin(&a.clk->cfl_min_bits, (unsigned long long)__double_as_longlong(m));
+      cfl_min(a.clk, m);
     }
   }
 }
