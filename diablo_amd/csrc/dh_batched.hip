@@ -549,18 +549,22 @@ int fail(int code, const std::string &msg) {
 }
 }  // namespace
 
-// the column tile (66.6 KB) is beyond the default dynamic-LDS limit
+// the column tile (66.6 KB) is beyond the default dynamic-LDS limit, which is
+// raised per device, at the first call on it
 hipError_t fft512_lds_limits() {
-  static hipError_t once = [] {
-    const void *k[] = {(const void *)k_fft512_cols<false, double2, 8>, (const void *)k_fft512_cols<true, double2, 8>,
-                       (const void *)k_fft512_cols<false, float2, 16>, (const void *)k_fft512_cols<true, float2, 16>};
-    for (const void *f : k) {
-      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
-      if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
-  }();
-  return once;
+  static bool raised[64] = {};
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+  std::lock_guard<std::mutex> lk(g_mu);
+  if (raised[dev]) return hipSuccess;
+  const void *k[] = {(const void *)k_fft512_cols<false, double2, 8>, (const void *)k_fft512_cols<true, double2, 8>,
+                     (const void *)k_fft512_cols<false, float2, 16>, (const void *)k_fft512_cols<true, float2, 16>};
+  for (const void *f : k)
+    if ((e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax)) != hipSuccess) return e;
+  raised[dev] = true;
+  return hipSuccess;
 }
 
 // planes per launch pair: all of them up to a grid's 2^32 threads
