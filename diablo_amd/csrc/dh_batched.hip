@@ -394,21 +394,23 @@ __global__ void __launch_bounds__(256) k_fft512_rows_fwd(const Sc<C> *__restrict
 template <class C>
 using AtReal __attribute__((aligned(sizeof(Sc<C>)))) = C;
 
-// x pass, inverse (the c2r of mpi.f:1600-1604, unnormalised), in place: rows
+// x pass, inverse (the c2r of mpi.f:1600-1604, unnormalised): rows
 // z, z+1 of the half spectra X, Y to x_n + i y_n = sum_k (X_k + i Y_k) e^{+2
 // pi i nk/512}, with X_{512-k} = conj X_k and the imaginary parts of X_0,
 // X_256 ignored as a c2r ignores them.  A row's 512 reals hold its X_k, k =
 // 1..255, as 256 complex values with (Re X_0, Re X_256) in the first, as the
-// z pass leaves them; a wave reads its two rows before it writes them.
+// z pass leaves them.  It runs in place (in == phys; a wave reads its two rows
+// before it writes them) or from planes elsewhere.
 template <class C>
-__global__ void __launch_bounds__(256) k_fft512_rows_inv(Sc<C> *phys, const C *__restrict__ tw, long long np) {
+__global__ void __launch_bounds__(256) k_fft512_rows_inv(const Sc<C> *in, Sc<C> *phys, const C *__restrict__ tw,
+                                                       long long np) {
   using S = Sc<C>;
   __shared__ C sm[4][kFftSlots];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const long long pair = (long long)blockIdx.x * 4 + w;
   if (pair >= np * (kFftN / 2)) return;
   S *oa = phys + 2 * pair * kFftN, *ob = oa + kFftN;
-  const AtReal<C> *ia = reinterpret_cast<const AtReal<C> *>(oa), *ib = reinterpret_cast<const AtReal<C> *>(ob);
+  const AtReal<C> *ia = reinterpret_cast<const AtReal<C> *>(in + 2 * pair * kFftN), *ib = ia + kFftN / 2;
   // Z_k = X_k + i Y_k for this lane's k = lane + 64 j < 256, and its mirror
   // Z_{512-k} = conj X_k + i conj Y_k through LDS to the lane that holds it
   // (each coefficient read once); Z_256 is lane 0's v[4]
@@ -603,17 +605,61 @@ static hipError_t fft512_forward_t(const void *phys, void *four, long long nplan
   return hipSuccess;
 }
 
+// mid: where the planes lie between the passes, chunk of them (null: in phys)
 template <class C>
-static hipError_t fft512_inverse_t(const void *four, void *phys, long long nplanes, hipStream_t st, const C *tw) {
-  for (long long p0 = 0; p0 < nplanes; p0 += kFftChunk) {
-    const long long np = std::min(kFftChunk, nplanes - p0);
-    Sc<C> *ph = (Sc<C> *)phys + p0 * kFftN * kFftN;
-    launch_fft512_cols<true, C>((const C *)four + p0 * kFftN * kFftK, nullptr, ph, tw, np, st);
-    hipLaunchKernelGGL(k_fft512_rows_inv<C>, dim3(fft512_row_blocks(np)), dim3(256), 0, st, ph, tw, np);
+static hipError_t fft512_inverse_t(const void *four, void *phys, long long nplanes, hipStream_t st, const C *tw,
+                                   Sc<C> *mid, long long chunk) {
+  for (long long p0 = 0; p0 < nplanes; p0 += chunk) {
+    const long long np = std::min(chunk, nplanes - p0);
+    Sc<C> *ph = (Sc<C> *)phys + p0 * kFftN * kFftN, *q = mid ? mid : ph;
+    launch_fft512_cols<true, C>((const C *)four + p0 * kFftN * kFftK, nullptr, q, tw, np, st);
+    hipLaunchKernelGGL(k_fft512_rows_inv<C>, dim3(fft512_row_blocks(np)), dim3(256), 0, st, q, ph, tw, np);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+// An inverse whose phys shares memory with its four: the column pass must not
+// write where other blocks still read, so the planes between the passes lie in
+// a static array, kOverlapPlanes at a time (33.6 MB on each device the library
+// runs on).  Calls on several streams take the array in turn; under capture,
+// where an event from outside cannot be waited for, a graph's calls are in
+// order with one another only.
+constexpr long long kOverlapPlanes = 16;
+__device__ __align__(256) double g_overlap_dev[kOverlapPlanes * kFftN * kFftN];
+static struct {
+  std::mutex mu;
+  void *at[64];         // the array's address on each device
+  hipEvent_t done[64];  // its last call there
+} g_overlap;
+
+static bool fft512_overlap(const void *four, const void *phys, long long nplanes, bool fp32) {
+  const size_t real = fp32 ? sizeof(float) : sizeof(double);
+  const char *f = (const char *)four, *p = (const char *)phys;
+  return f < p + nplanes * kFftN * kFftN * real && p < f + nplanes * kFftN * kFftK * 2 * real;
+}
+
+template <class C>
+static hipError_t fft512_inverse_overlap(const void *four, void *phys, long long nplanes, hipStream_t st, const C *tw) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);  // below 64: twiddles has checked it
+  if (e != hipSuccess) return e;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if ((e = hipStreamIsCapturing(st, &cap)) != hipSuccess) return e;
+  const bool order = cap == hipStreamCaptureStatusNone;
+  std::lock_guard<std::mutex> lk(g_overlap.mu);
+  void *&mid = g_overlap.at[dev];
+  hipEvent_t &ev = g_overlap.done[dev];
+  if (!mid && (e = hipGetSymbolAddress(&mid, HIP_SYMBOL(g_overlap_dev))) != hipSuccess) return e;
+  if (order && ev && (e = hipStreamWaitEvent(st, ev, 0)) != hipSuccess) return e;
+  if (order && !ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
+  e = fft512_inverse_t<C>(four, phys, nplanes, st, tw, static_cast<Sc<C> *>(mid), kOverlapPlanes);
+  if (order) {
+    const hipError_t r = hipEventRecord(ev, st);
+    if (e == hipSuccess) e = r;
+  }
+  return e;
 }
 
 static hipError_t fft512_transform(bool inverse, const void *src, void *dst, long long nplanes, bool fp32,
@@ -625,8 +671,12 @@ static hipError_t fft512_transform(bool inverse, const void *src, void *dst, lon
   if (e != hipSuccess) return e;
   const float2 *t32 = static_cast<const float2 *>(tw);
   const double2 *t64 = static_cast<const double2 *>(tw);
+  if (inverse && fft512_overlap(src, dst, nplanes, fp32))
+    return fp32 ? fft512_inverse_overlap<float2>(src, dst, nplanes, st, t32)
+                : fft512_inverse_overlap<double2>(src, dst, nplanes, st, t64);
   if (inverse)
-    return fp32 ? fft512_inverse_t<float2>(src, dst, nplanes, st, t32) : fft512_inverse_t<double2>(src, dst, nplanes, st, t64);
+    return fp32 ? fft512_inverse_t<float2>(src, dst, nplanes, st, t32, nullptr, kFftChunk)
+                : fft512_inverse_t<double2>(src, dst, nplanes, st, t64, nullptr, kFftChunk);
   return fp32 ? fft512_forward_t<float2>(src, dst, nplanes, st, t32) : fft512_forward_t<double2>(src, dst, nplanes, st, t64);
 }
 

@@ -332,7 +332,11 @@ int dh_fft512_xz_to_fourier_dev(const void *phys, void *four, int64_t nplanes, i
  * the backward complex transform along z, then complex-to-real along x
  * (the imaginary parts of kx = 0 and 256 ignored, as a c2r ignores them).
  * four is left unchanged (the reference's transform destroys its input);
- * the planes between the passes are held in phys.  Nothing is allocated. */
+ * the planes between the passes are held in phys.  Nothing is allocated.
+ * phys may be four, or start before it in the same memory (of four, what phys
+ * does not cover stays): the planes between the passes then go 16 at a time
+ * through a static array of 33.6 MB per device, which calls take in turn; a
+ * captured call of this kind must not run beside others of its kind. */
 int dh_fft512_xz_to_physical_dev(const void *four, void *phys, int64_t nplanes, int32_t fp32, void *stream);
 /* The same under the name that callers who cannot allocate device memory
  * (code under stream capture, tight serving loops, harnesses that forbid

@@ -11,6 +11,7 @@
 #include <map>
 #include <set>
 #include <utility>
+#include <vector>
 
 namespace {
 struct Dim3 {
@@ -23,12 +24,24 @@ std::map<std::pair<int, const void *>, void *> g_symbols;
 Dim3 g_grid, g_block;
 size_t g_lds;
 void *g_stream;
+int g_nargs = 0;
+std::vector<uint64_t> g_log;
 void *handle(void **p) { return *p = calloc(1, 8); }
 }  // namespace
 
 extern "C" {
 void host_set_device(int d) { g_device = d; }
 void host_refuse_launches(int on) { g_refuse_launches = on != 0; }
+// the first nargs arguments (8 bytes each) of every launch from now on
+void host_record(int nargs) {
+  g_nargs = nargs;
+  g_log.clear();
+}
+int host_recorded(uint64_t *out, int most) {
+  int n = 0;
+  for (; n < most && n < (int)g_log.size(); ++n) out[n] = g_log[n];
+  return (int)g_log.size();
+}
 
 int hipGetDevice(int *d) {
   *d = g_device;
@@ -65,8 +78,9 @@ int hipFuncSetAttribute(const void *f, int, int) {
   g_raised.insert({g_device, f});
   return 0;
 }
-int hipLaunchKernel(const void *f, Dim3, Dim3, void **, size_t lds, void *) {
+int hipLaunchKernel(const void *f, Dim3, Dim3, void **args, size_t lds, void *) {
   if (g_refuse_launches || (lds > 65536 && !g_raised.count({g_device, f}))) return g_last = 1;
+  for (int i = 0; i < g_nargs; ++i) g_log.push_back(*static_cast<uint64_t *>(args[i]));
   return 0;
 }
 unsigned __hipPushCallConfiguration(Dim3 g, Dim3 b, size_t lds, void *st) {
