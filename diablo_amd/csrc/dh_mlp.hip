@@ -121,7 +121,9 @@ constexpr int kPartLd = (kMlpNP + 1 + 3) / 4 * 4;  // floats per block of partia
 __global__ void __launch_bounds__(kTrThreads, 2) k_mlp_train(const bf16x8 *pk, const float *P,
                                                            const float *__restrict__ x, const float *__restrict__ t,
                                                            long long N, float inv_n, float *__restrict__ part) {
-  __shared__ __bf16 act[kTrRows * kTrLd];
+  __shared__ alignas(bf16x8) __bf16 act[kTrRows * kTrLd];
+  static_assert(__alignof__(act) >= alignof(bf16x8) && kTrLd * sizeof(__bf16) % alignof(bf16x8) == 0,
+                "a row is read in pieces of 8 values");
   __shared__ float wloss[kTrThreads / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
