@@ -290,8 +290,12 @@ __device__ __forceinline__ void fft_stage(C *A, const FftStage &st, int N, int n
   lds_barrier();
 }
 
+// Always inlined: with as many callers as it has, the compiler takes it out of
+// line in some, and the nonlinear pass's 256 registers per lane do not hold a
+// call's besides (4 spilled; 280 B of scratch in the batched form).
 template <bool INV, bool COLS, bool DIT, class C>
-__device__ void lds_fft(C *A, const FftPlan &pl, int ntrans, unsigned long long fnt, int ls, const C *tw) {
+__device__ __forceinline__ void lds_fft(C *A, const FftPlan &pl, int ntrans, unsigned long long fnt, int ls,
+                                        const C *tw) {
 #pragma unroll 1
   for (int s = 0; s < pl.nst; ++s) {
     const FftStage &st = DIT ? pl.dit[s] : pl.dif[s];
