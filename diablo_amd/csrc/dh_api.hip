@@ -705,10 +705,16 @@ int dh_set_mixed_precision(dh_ctx *h, int32_t on) {
     HIPCHK(dalloc(&c.rphys32, n));
   }
   c.mixed = (on != 0);
-  drop_graphs(c);  // the captured steps launch the other form's kernels
   set_solve_segments(c);
   // the solve tables are laid out by segments, and each form has its pivots
-  return c.grid_set ? rebuild_tables(c) : DH_OK;
+  const int r = c.grid_set ? rebuild_tables(c) : DH_OK;
+  if (r != DH_OK) {  // the form stays that of the tables
+    c.mixed = !c.mixed;
+    set_solve_segments(c);
+    return r;
+  }
+  drop_graphs(c);  // the captured steps launch the other form's kernels
+  return DH_OK;
 }
 
 int dh_mixed_precision(dh_ctx *h) { return h ? (h->c.mixed ? 1 : 0) : DH_EARG; }

@@ -137,7 +137,8 @@ int dh_time_step(dh_ctx *ctx, int32_t nsteps);
  * CFTH), the accumulation of CF, the RK combination, the Crank-Nicolson and
  * pressure-Poisson solves and COURANT stay FP64.  on = 0 returns to the FP64
  * drop-in path.  The first switch allocates two FP32 physical arrays of
- * (NY+2)*NX*NZ*(3+N_TH) values. */
+ * (NY+2)*NX*NZ*(3+N_TH) values.  Every switch waits for the context's stream
+ * and makes the solve tables of the new form; on an error the form stays. */
 int dh_set_mixed_precision(dh_ctx *ctx, int32_t on);
 /* 1 when the mixed form is on, 0 when not. */
 int dh_mixed_precision(dh_ctx *ctx);

@@ -1,6 +1,6 @@
 """The library's host code against a stand-in for the HIP runtime's host
 calls (tests/hip_host.cpp; no GPU): what its entry points do on a second
-device and with buffers that share memory."""
+device, with buffers that share memory and where a launch is refused."""
 import os
 import subprocess
 import sys
@@ -67,4 +67,19 @@ for i, ((src, _, mid), (rin, out, _)) in enumerate(zip(cols, rows)):
     assert mid + (p1 - p0) * plane_out <= four - ahead or mid >= end
     assert out + (p1 - p0) * plane_out <= four + p1 * plane_in
 assert p1 == n
+""")
+
+
+def test_refused_tables_leave_the_form(host_runtime):
+    """dh_set_mixed_precision where the other form's solve tables cannot be made."""
+    _run(host_runtime, """
+p, gy, ic = configs.CONFIGS["small_case"]()
+ch = channel.Channel(p, gy)
+for form in (1, 0):
+    host.host_refuse_launches(1)
+    assert lib.dh_set_mixed_precision(ch.h, form) != 0
+    assert lib.dh_mixed_precision(ch.h) == 1 - form, "switched without its tables"
+    host.host_refuse_launches(0)
+    assert lib.dh_set_mixed_precision(ch.h, form) == 0
+    assert lib.dh_mixed_precision(ch.h) == form
 """)
