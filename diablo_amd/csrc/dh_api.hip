@@ -135,7 +135,7 @@ hipError_t dalloc(T **p, size_t count) {
 void free_all(Ctx &c) {
   void *ptrs[] = {c.tw_row, c.tw_col, c.tw_real, c.posr, c.posrd, c.posz, c.posc, c.kx, c.kz, c.kx2, c.kz2, c.d_dy, c.d_dyf, c.d_gyf, c.d_rdy, c.d_rdyf, c.cu[0], c.cu[1],
                   c.cu[2], c.cp, c.cf[0], c.cf[1], c.cf[2], c.cth, c.cfth, c.phi, c.uphys, c.rphys, c.rd_ta,
-                  c.rd_tb, c.clock, c.fac.pf, c.fac.pb, c.fac.tl, c.fac.tb, c.fac.tc, c.fac.tr, c.fac.isbc, c.rd_tr, c.fac.vconst, c.rd_l, c.rd_u, c.stats, c.cun[0], c.cun[1], c.cun[2], c.uphys32, c.rphys32, c.fac.bcl, c.fac.bcd, c.fac.bcu, c.nut, c.cul, c.les_four, c.les_phys, c.sgs, c.les_wk, c.d_lesw, c.d_mlp_p, c.d_mlp_pk, c.les_feat, c.gp_scratch};
+                  c.rd_tb, c.clock, c.fac.pf, c.fac.pb, c.fac.pw, c.fac.tl, c.fac.tb, c.fac.tc, c.fac.tr, c.fac.isbc, c.rd_tr, c.fac.vconst, c.rd_l, c.rd_u, c.stats, c.cun[0], c.cun[1], c.cun[2], c.uphys32, c.rphys32, c.fac.bcl, c.fac.bcd, c.fac.bcu, c.nut, c.cul, c.les_four, c.les_phys, c.sgs, c.les_wk, c.d_lesw, c.d_mlp_p, c.d_mlp_pk, c.les_feat, c.gp_scratch};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c.step_graph) (void)hipGraphExecDestroy(c.step_graph);
@@ -355,6 +355,7 @@ int dh_create(const dh_params *p, dh_ctx **out) {
   ACHK(dalloc(&c.clock, 1));
   ACHK(dalloc(&c.fac.pf, 3 * (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.pb, 3 * (size_t)c.nfields * nyy));
+  ACHK(dalloc(&c.fac.pw, 3 * (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.tl, 3 * (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.tb, 3 * (size_t)c.nfields * nyy));
   ACHK(dalloc(&c.fac.tc, 3 * (size_t)c.nfields * nyy));

@@ -111,6 +111,7 @@ struct CourantArgs {
 struct RealFactors {
   double *tl, *tb, *tc, *tr;  // [rk][field][row] Thomas multipliers, pivots, upper diagonal, 1/pivots
   double *pf, *pb;            // [rk][field][row] segment carry factors of the two sweeps
+  double *pw;                 // [rk][field][row] weight of a row in its segment's first value (FP64 form)
   int *isbc;                  // [field][row] 1: row takes a constant right-hand side
   double *vconst;             // [field][row]
   double *bcl, *bcd, *bcu;    // [field][row] coefficients of the boundary rows (isbc = 1)

@@ -1329,9 +1329,10 @@ __host__ __device__ inline void real_row(const FactorIn &in, int f, double temp1
 // Tables of the shared matrix of (rk, field), one block each: rows from
 // real_row, the forward elimination of THOMAS_REAL_MPI (mpi.f:630-703) in
 // its operation order (multipliers TL, pivots TB, upper diagonal TC, 1/TB),
-// and the carry factors of the segmented sweeps of k_solve_seg:
+// and the carry factors of the segmented sweeps (k_solve_cols, k_solve_seg):
 //   PF_J = prod_{i=a..J} TL_i          (a: first row of J's segment)
 //   PB_J = prod_{i=J..b-1} -TC_i/TB_i  (b-1: last row of J's segment)
+//   PW_J = prod_{i=a..J-1} -TC_i/TB_i / TB_J  (FP64 form)
 // The constant right-hand sides of the boundary rows and the rows'
 // coefficients (dt independent) are written by the rk=0 blocks.
 __device__ __forceinline__ void cn_tables_body(const Clock *clk, const FactorIn &in, const RealFactors &fac, int blk) {
@@ -1441,7 +1442,9 @@ __device__ __forceinline__ void cn_tables_body(const Clock *clk, const FactorIn 
   }
   __syncthreads();
   // the carry factors of a row: the products of its segment's multipliers up
-  // to it, and of the backward quotients from its segment's end down to it
+  // to it, and of the backward quotients from its segment's end down to it; and
+  // its weight in the segment's first value
+  const long long o = ((long long)rk * in.nfields + f) * nrow;
   for (int J = threadIdx.x; J < nrow; J += blockDim.x) tr[J] = (tb[J] != 0.0) ? -c[J] / tb[J] : 0.0;
   __syncthreads();
   for (int J = threadIdx.x; J < nrow; J += blockDim.x) {
@@ -1452,9 +1455,13 @@ __device__ __forceinline__ void cn_tables_body(const Clock *clk, const FactorIn 
     double g = tr[s1];
     for (int i = s1 - 1; i >= J; --i) g = tr[i] * g;
     pb[J] = g;
+    if (!in.serial) {
+      double w = (tb[J] != 0.0) ? 1.0 / tb[J] : 0.0;
+      for (int i = J - 1; i >= s0; --i) w = tr[i] * w;
+      fac.pw[o + J] = w;
+    }
   }
   __syncthreads();
-  const long long o = ((long long)rk * in.nfields + f) * nrow;
   for (int i = threadIdx.x; i < nrow; i += blockDim.x) {
     fac.tl[o + i] = tl[i];
     fac.tb[o + i] = tb[i];
@@ -1479,19 +1486,22 @@ __global__ void __launch_bounds__(256) k_cn_tables_b(const CnArgs *__restrict__ 
 // Real Crank-Nicolson solves (channel.f:771-1029; the explicit half of the
 // y-viscous term is already in R, added in Fourier space by k_nonlinear) and
 // the CFL minimum of COURANT (courant.f:34-43).  THOMAS_REAL_MPI's sweeps
-// (mpi.f:630-703, 767-809) run on columns split into NS segments of
-// seg_rows rows, each held in the registers of one lane (lane = segment *
-// 64/NS + column):
-//   forward:  each segment sweeps from a zero carry, h_J = d_J + TL_J h_{J-1};
-//             the carries g_{a-1} pass up the segments by shuffles, and
-//             g_J = h_J + PF_J g_{a-1};
-//   backward: each segment sweeps from a zero carry, y_J = (g_J - TC_J
-//             y_{J+1}) / TB_J (quotient from 1/TB_J, the same double as the
-//             division); the carries x_b pass down, and x_J = y_J + PB_J x_b.
-// (k_solve_cols: through LDS.)
-// The first segment's forward values and the last segment's backward values
-// are the reference's own; the others differ from a single sweep by the
-// rounding of the carry terms.
+// (mpi.f:630-703, 767-809) run on columns split into segments of seg_rows
+// rows, each held in the registers of one lane (k_solve_seg: lane = segment *
+// 64/NS + column; k_solve_cols: thread = segment * 32 + column):
+//   forward:  each segment sweeps from a zero carry, h_J = d_J + TL_J h_{J-1},
+//             and with g_end = h_end + PF_end g_{a-1} the carries g_{a-1} pass
+//             up the segments;
+//   backward: a segment's first value is y_a + PB_a x_b with y_a from a zero
+//             carry, y_J = (g_J - TC_J y_{J+1}) / TB_J, and so the carries x_b
+//             pass down.
+// k_solve_cols then repeats a segment's rows from its carries in the
+// reference's own operations (the quotient from 1/TB_J, the same double as the
+// division), so only the carries are composed.  k_solve_seg adds the carry
+// terms PF_J g_{a-1} and PB_J x_b to the rows of the zero carry, a rounding more
+// in each: with 16 short segments that put the error of CP against 64 bits at
+// 7.1e-13 where a single sweep has 5.0e-13 and the repeated rows 4.7e-13 (64 x 65
+// x 4 shear layer, one step).
 // ---------------------------------------------------------------------------
 struct SolveArgs {
   Geo g;
@@ -1663,17 +1673,21 @@ constexpr int kColCols = 32;  // columns per block
 // The FP64 solve: a block takes 32 neighbouring columns in 16 segments of up to
 // SR rows, one thread per segment and column (columns fastest, so that a wave's
 // loads and stores are whole 256-byte pieces of two rows), and the carries cross
-// the segments through LDS.  It is bound by memory for many columns and by
-// the chain of rows for few, so rows stay few per thread: with a column in 4 or
-// 8 lanes of 36 rows it took 174 us at 256 x 193 x 256 (1.2 GB; 127 in this form),
-// 26 at 128 x 129 x 128 (25), 19.7 at 256 x 257 x 4 (11.9) and 13.6 at
-// 64 x 65 x 4 (5.3).  32 segments take 10.4, but 199 at 256 x 193 x 256; 16
-// columns a block 139 there, 64 columns 145.
+// the segments through LDS.  The carries' zero-carry values take one
+// multiply-add a row: h in a sweep before the rows', y_a as the sum PW_J g_J
+// (PW_J = prod_{i=a..J-1} -TC_i/TB_i / TB_J) beside them; y_a by a backward sweep
+// of its own took 12.2 us at 256 x 257 x 4 (11.2 this way).  It is bound by memory
+// for many columns and by the chain of rows for few, so rows stay few per
+// thread: 143 us at 256 x 193 x 256 (0.61 GB), 26 at 128 x 129 x 128, 11.2 at
+// 256 x 257 x 4 and 5.3 at 64 x 65 x 4; with a column in 4 or 8 lanes of 36 rows
+// 174, 26, 19.7 and 13.6.  With carry terms added to the rows instead, 125, 25,
+// 12.1 and 5.4, and in that form 32 segments took 199 us at 256 x 193 x 256, 16
+// columns a block 139, 64 columns 145.
 template <int SR>
 __device__ __forceinline__ void solve_cols_body(const SolveArgs &a) {
 #pragma clang fp contract(off)
   constexpr int NSEG = kColSegs, CB = kColCols, NR = NSEG * SR, NT = NSEG * CB;
-  __shared__ double TL[NR], TB[NR], TC[NR], TR[NR], PF[NR], PB[NR], VC[NR];
+  __shared__ double TL[NR], TB[NR], TC[NR], TR[NR], PW[NR], VC[NR], PF[NSEG], PB[NSEG];
   __shared__ int IB[NR];
   __shared__ double H[NSEG * CB];
   __shared__ double red[NT / 64];
@@ -1693,8 +1707,7 @@ __device__ __forceinline__ void solve_cols_body(const SolveArgs &a) {
   double v[SR];
 #pragma unroll
   for (int q = 0; q < SR; ++q) v[q] = Rb[ro_(min(r0 + q, nrow - 1))];
-  // rows beyond a segment's: the forward carry passes through them (TL = 1),
-  // the backward sweep starts from zero in them
+  // rows beyond a segment's change nothing: TL = 1, the rest zero
   const long long to = ((long long)a.rk * a.nfields + f) * nrow, fo = (long long)f * nrow;
   for (int e = threadIdx.x; e < NR; e += NT) {
     const int s = e / SR, q = e - s * SR, i = s * sr + q;
@@ -1703,43 +1716,50 @@ __device__ __forceinline__ void solve_cols_body(const SolveArgs &a) {
     TB[e] = in ? a.fac.tb[to + i] : 1.0;
     TC[e] = in ? a.fac.tc[to + i] : 0.0;
     TR[e] = in ? a.fac.tr[to + i] : 1.0;
-    PF[e] = in ? a.fac.pf[to + i] : 0.0;
-    PB[e] = in ? a.fac.pb[to + i] : 0.0;
+    PW[e] = in ? a.fac.pw[to + i] : 0.0;
     VC[e] = in ? a.fac.vconst[fo + i] : 0.0;
     IB[e] = in ? a.fac.isbc[fo + i] : 1;
   }
+  if (threadIdx.x < NSEG) {  // the carry factors over whole segments
+    const int i0 = threadIdx.x * sr, i1 = i0 + sr - 1;
+    PF[threadIdx.x] = (i1 < nrow) ? a.fac.pf[to + i1] : 0.0;
+    PB[threadIdx.x] = (i0 < nrow) ? a.fac.pb[to + i0] : 0.0;
+  }
   __syncthreads();
   const int t0 = seg * SR;
-  // right-hand sides (the boundary constant or R), forward from a zero carry
-  double hp = 0.0;
+  // right-hand sides: the boundary constant or R
+#pragma unroll
+  for (int q = 0; q < SR; ++q) v[q] = IB[t0 + q] ? VC[t0 + q] : v[q];
+  // forward from a zero carry, for the segment's end (TL = 1 passes it through
+  // the rows beyond the segment's)
+  double h = 0.0;
+#pragma unroll
+  for (int q = 0; q < SR; ++q) h = fma(TL[t0 + q], h, v[q]);
+  H[threadIdx.x] = h;
+  __syncthreads();
+  // g_in(s) = g_end(s-1), g_end = h_end + PF g_in, and the rows from it
+  double gx = 0.0;
+  for (int s = 0; s < seg; ++s) gx = fma(PF[s], gx, H[s * CB + cl]);
+  double y = 0.0;  // the segment's first value from a zero carry above it
 #pragma unroll
   for (int q = 0; q < SR; ++q) {
-    const double d = IB[t0 + q] ? VC[t0 + q] : v[q];
-    hp = d + TL[t0 + q] * hp;
-    v[q] = hp;
+    gx = v[q] + TL[t0 + q] * gx;
+    v[q] = gx;
+    y = fma(PW[t0 + q], gx, y);
   }
-  H[threadIdx.x] = hp;
   __syncthreads();
-  // g_in(s) = g_end(s-1), g_end = h_end + PF_end g_in
-  double gin = 0.0;
-  for (int s = 0; s < seg; ++s) gin = H[s * CB + cl] + PF[s * SR + sr - 1] * gin;
-#pragma unroll
-  for (int q = 0; q < SR; ++q) v[q] = (seg == 0) ? v[q] : v[q] + PF[t0 + q] * gin;
-  // backward from a zero carry
-  double yn = 0.0;
+  H[threadIdx.x] = y;  // zero where the segment is empty
+  __syncthreads();
+  // x_in(s) = x_start(s+1), x_start = y_start + PB x_in, and the rows from it
+  double x = 0.0;
+  for (int s = NSEG - 1; s > seg; --s) x = fma(PB[s], x, H[s * CB + cl]);
 #pragma unroll
   for (int q = SR - 1; q >= 0; --q) {
     const double b = TB[t0 + q];
-    const double y = (b != 0.0) ? div_by_recip(v[q] - TC[t0 + q] * yn, b, TR[t0 + q]) : 0.0;
-    v[q] = y;
-    yn = (q < nr) ? y : 0.0;
+    const double xq = (b != 0.0) ? div_by_recip(v[q] - TC[t0 + q] * x, b, TR[t0 + q]) : 0.0;
+    x = (q < nr) ? xq : x;
+    v[q] = x;
   }
-  __syncthreads();
-  H[threadIdx.x] = (nr > 0) ? yn : 0.0;
-  __syncthreads();
-  // x_in(s) = x_start(s+1), x_start = y_start + PB_start x_in
-  double xin = 0.0;
-  for (int s = NSEG - 1; s > seg; --s) xin = H[s * CB + cl] + PB[s * SR] * xin;
   const bool cour = a.courant && f < 3;
   const double dxf = (f == 0) ? a.dx : a.dz;
   double dtmin = __longlong_as_double(0x7FF0000000000000ll), xmax = 0.0;
@@ -1747,14 +1767,13 @@ __device__ __forceinline__ void solve_cols_body(const SolveArgs &a) {
 #pragma unroll
   for (int q = 0; q < SR; ++q) {
     const int i = r0 + q;
-    const double x = (r0 + sr >= nrow) ? v[q] : v[q] + PB[t0 + q] * xin;
     if (live && q < nr && i >= wlo && i <= whi) {
-      Ub[ro_(i)] = x;
+      Ub[ro_(i)] = v[q];
       if (cour && i >= 1 && i <= NY) {
         if (f == 1)
-          dtmin = fmin(dtmin, a.cfl * g.dy[i] / fabs(x));
+          dtmin = fmin(dtmin, a.cfl * g.dy[i] / fabs(v[q]));
         else
-          xmax = fmax(xmax, fabs(x));
+          xmax = fmax(xmax, fabs(v[q]));
       }
     }
   }
