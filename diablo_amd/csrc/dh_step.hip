@@ -1363,8 +1363,9 @@ __device__ __forceinline__ void cn_tables_body(const Clock *clk, const FactorIn 
   // The forward elimination, B_J = D_J - L_J U_{J-1} / B_{J-1}, is a
   // recurrence through a division.  One thread takes 0.19 us a row, and the
   // tables outlast REM_DIV in the launch the two share (128 x 129 x 128: 34 us
-  // with one thread, 17.0 with the scan below, 16.9 without tables).  The rows of these systems have |D| = S + |L| + |U| with
-  // S >= 0 and -L D, -U D >= 0; then so has every pivot, |B_J| = s_J + |U_J|, and
+  // with one thread, 17.0 with the scan below, 17.1 without tables).  The rows
+  // of these systems have |D| = S + |L| + |U| with S >= 0 and -L D, -U D >= 0;
+  // then so has every pivot, |B_J| = s_J + |U_J|, and
   //   s_J = S_J + |L_J| s_{J-1} / (s_{J-1} + |U_{J-1}|),
   // a 2 x 2 matrix on s = n/d whose entries are not negative: products of such
   // matrices don't cancel.  The first wave composes those of its lanes' rows by
@@ -1415,11 +1416,19 @@ __device__ __forceinline__ void cn_tables_body(const Clock *clk, const FactorIn 
       }
       bp = __shfl_up(p00 / p10, 1);  // s of the row below this lane's
       if (lane > 0 && r0 < nrow) bp = copysign(bp + fabs(c[r0 - 1]), b[r0 - 1]);
-      for (int J = r0; J < r1; ++J) {
-        const double m = J > 0 ? -a[J] / bp : 0.0;
-        bp = J > 0 ? b[J] + m * c[J - 1] : b[0];
-        tl[J] = m;
-        tb[J] = bp;
+      // the rows from it; twice, as the products round more often than the
+      // recurrence does (up to 10 units of the last place in the multiplier of a
+      // lane's first row, where its own rounding is 2) and a pivot forgets what
+      // it started from: the second time a lane starts from the pivot that the
+      // lane below it ended on
+      for (int pass = 0; pass < 2; ++pass) {
+        for (int J = r0; J < r1; ++J) {
+          const double m = J > 0 ? -a[J] / bp : 0.0;
+          bp = J > 0 ? b[J] + m * c[J - 1] : b[0];
+          tl[J] = m;
+          tb[J] = bp;
+        }
+        if (pass == 0) bp = __shfl_up(bp, 1);
       }
     } else if (lane == 0) {
       bp = b[0];

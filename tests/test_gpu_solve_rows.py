@@ -46,3 +46,12 @@ def _substep(dor, ny, bc):
 def test_rows_are_the_sweeps_own(oracle_mod, ny):
     print(f"[solve rows] ny={ny}", flush=True)
     _substep(oracle_mod, ny, 0)
+
+
+@pytest.mark.parametrize("ny", [40, 65, 127, 129, 192, 257])
+def test_pivots_are_the_recurrence_own(oracle_mod, ny):
+    """Free-slip walls: the wall row's multiplier is 1/pivot of the row below
+    it, so the pivot that a lane of the tables' scan starts from shows in the
+    wall value; at NY = 129 and 192 the row is a lane's first."""
+    print(f"[solve rows] free-slip ny={ny}", flush=True)
+    _substep(oracle_mod, ny, 1)
