@@ -68,9 +68,6 @@ struct Clock {
   int pad;
 };
 
-// Parallel-cyclic-reduction tables of the y-implicit (Crank-Nicolson)
-// matrices, one set per RK substep and field; with LES off each matrix
-// depends only on j, so every (x,z) column of a field shares it.
 // Most rows of one column held by one lane of the mixed form's Crank-Nicolson
 // solve; a column is split into 4 (NY+2 <= 144) or 8 such segments.
 constexpr int kSegRows = 36;
@@ -93,10 +90,11 @@ constexpr int kRowK2 = 6;
 // than one context's need (a smaller context created later would otherwise
 // lower it under a larger one).
 constexpr int kLdsMax = 160 * 1024;
-// Planes too large for LDS (dh_create sets Ctx::gp) are transformed in
-// chunks staged through LDS, the plane between the row and the column pass
-// held in a scratch slot in device memory: kGpSlots slots per stream half,
-// one per block of the persistent large-plane kernels (kGpThreads threads).
+// Planes too large for LDS (dh_create sets Ctx::gp) run as pencils up to 512
+// points a side (Ctx::pencil); longer ones are transformed in chunks staged
+// through LDS, the plane between the row and the column pass held in a scratch
+// slot in device memory: kGpSlots slots per stream half, one per block of the
+// persistent large-plane kernels (kGpThreads threads).
 constexpr int kGpSlots = 256, kGpThreads = 1024;
 
 struct CourantArgs {
@@ -209,9 +207,10 @@ struct Ctx {
   double mlp_ts = 1.0, mlp_ls = 1.0, mlp_nus = 1.0;  // time scale, length scale, NU_T scale
   double *les_feat = nullptr;
   // planes too large for LDS: kGpSlots scratch slots for the main stream's
-  // kernels and kGpSlots for the branch's, gp_slot complex values each (a
-  // plane between the row and the column pass, NZ rows of the NKX+1 kept x
-  // modes, then the nonlinear pass's accumulators of the PF modes)
+  // persistent kernels and kGpSlots for the branch's, gp_slot complex values
+  // each (a plane between the row and the column pass, NZ rows of the NKX+1 kept
+  // x modes, then the nonlinear pass's accumulators of the PF modes); the
+  // pencils take all of it for the planes between their passes
   bool gp = false;
   double2 *gp_scratch = nullptr;
   bool pencil = false;          // large planes run as pencils (NX, NZ <= kPencilMax)
@@ -221,11 +220,11 @@ struct Ctx {
 inline double2 *gp_base(const Ctx &c, hipStream_t st) {
   return c.gp_scratch + (st == c.branch ? (long long)kGpSlots * c.gp_slot : 0LL);
 }
-// The large-plane kernels' LDS (all of a CU's: one block of 16 waves per
-// CU, 4 per SIMD, which their launch bounds keep to 128 VGPRs; against two
-// blocks of half the size, the larger chunks halve the barriers per plane
-// and the step at 256 x 193 x 256 takes 7.4 instead of 7.9 ms): the
-// transform tables (load_tables_at), in double2 units rounded up, then the
+// The persistent large-plane kernels' LDS (all of a CU's: one block of 16 waves
+// per CU, 4 per SIMD, which their launch bounds keep to 128 VGPRs; against two
+// blocks of half the size, the larger chunks halve the barriers per plane:
+// 7.4 instead of 7.9 ms a step at 256 x 193 x 256, which these kernels took
+// before the pencils): the transform tables (load_tables_at), in double2 units rounded up, then the
 // staging buffer of the row and column passes.
 constexpr int kGpLds = kLdsMax;
 __host__ __device__ inline int gp_table_elems(const Geo &g) {
@@ -238,8 +237,8 @@ constexpr int kPencilCols = 8;
 constexpr int kPencilThreads = 512;
 // (a column block of the nonlinear pass at NZ = 512 fills the LDS, 150 KB; longer
 // rows and columns run on the persistent kernels above, planes that fit LDS on
-// the plane kernels: 128 x 129 x 128 takes 1.31 ms for two steps there and
-// 1.95 as pencils)
+// the plane kernels: 128 x 129 x 128 takes 0.97 ms for two steps there and
+// 1.72 as pencils)
 constexpr int kPencilMax = 512;
 __host__ __device__ inline int pencil_stride(const Geo &g) {
   return (g.nkx1 + kPencilCols - 1) / kPencilCols * kPencilCols;

@@ -932,7 +932,8 @@ __global__ void __launch_bounds__(kNlSmallThreads, 4) k_nonlinear_small_b(const 
 //
 // What bounds it: per 96 planes of 256 x 256 the products take 156 us (the
 // LDS stages of eight row transforms per row; 0.36 GB from and to memory),
-// the combination 204 (0.58 GB; the modes' loads, 16 waves on a CU) and the
+// the combination 204 (0.58 GB; the modes' loads, 16 waves on a CU; 12 of its
+// 127 registers spill) and the
 // inverse rows 67 (0.23 GB).  One block per CU that keeps a plane's transform
 // to itself (nonlinear_pass_gp), with the plane and CF's accumulators passing
 // through memory between all its passes, took 1.74 ms a substep at 256 x 193 x
@@ -1903,7 +1904,7 @@ __global__ void __launch_bounds__(256) k_rem_div_factors(RemDivArgs a) {
 // set from row 2.
 //
 // What bounds it: memory where the modes fill the chip (71 MB in 16.5 us at
-// 128 x 129 x 128, 0.50 GB in 141 us at 256 x 193 x 256), the chain of loads,
+// 128 x 129 x 128, 0.43 GB in 142 us at 256 x 193 x 256), the chain of loads,
 // two scans and stores where they do not (13.4 us at 256 x 257 x 4, 9.2 at
 // 64 x 97 x 64).  With eight lanes sweeping 17 rows each (NY <= 137) or one
 // lane all rows beyond, operands in LDS and the other waves idle, the same
@@ -2702,7 +2703,7 @@ static hipError_t launch_nonlinear_range(Ctx &c, int rk, int c0, int c1, hipStre
   a.j0 = jlo;
   const dim3 grid(jhi - jlo + 1, c1 - c0);
   if (c.pencil) return launch_nonlinear_pencil(c, a, c0, c1, jlo, jhi, st);
-  if (c.gp) {  // planes beyond LDS (FP64, no LES)
+  if (c.gp) {  // longer rows or columns than the pencils take
     if (c.recording) return hipErrorNotSupported;
     double2 *gp = gp_base(c, st);
     long long slot = c.gp_slot;
@@ -2716,12 +2717,13 @@ static hipError_t launch_nonlinear_range(Ctx &c, int rk, int c0, int c1, hipStre
 }
 
 // Whether the substep runs flat: each phase one launch over all fields on
-// the context stream.  Planes in LDS do: with U3's nonlinear pass, solve
-// and transform on a branch beside U1's and U2's, the branch's solve and
+// the context stream.  Planes in LDS and pencils do: with U3's nonlinear pass,
+// solve and transform on a branch beside U1's and U2's, the branch's solve and
 // transform wait for its pass, and the fork and join cost 6-10 us each
-// (config 1: 0.638 ms per step flat against 0.657 with the branch).  The
-// large-plane kernels keep the branch (256 x 193 x 256: 7.2 ms per step
-// against 7.55 flat).
+// (128 x 129 x 128 in the kernels before these: 0.638 ms per step flat against
+// 0.657 with the branch).  The persistent kernels of longer rows and columns
+// keep the branch (7.2 ms per step against 7.55 flat at 256 x 193 x 256, which
+// they took before the pencils).
 static bool flat_substep(const Ctx &c) { return !c.gp || c.pencil; }
 
 
@@ -3380,8 +3382,8 @@ hipError_t join_side(Ctx &c) {
   return kwait(c, c.stream, 3);  // ev_join
 }
 
-// One substep.  With planes in LDS each phase is one launch over all fields
-// on the context stream (flat_substep).  On the large-plane path the
+// One substep.  With planes in LDS or pencils each phase is over all fields
+// on the context stream (flat_substep).  With the persistent kernels the
 // nonlinear pass of U1 and U2 runs on the context stream and the last
 // velocity component's nonlinear pass, solve and transform back (then the
 // scalars' nonlinear pass and solve) as a branch beside it and U1's and
@@ -3425,7 +3427,7 @@ hipError_t launch_substep(Ctx &c, int rk, int bnd_end, int bnd_begin, bool tick)
     SCHK(fuse_tables ? launch_rem_div_cn(c, rk, bnd_end, bnd_begin) : launch_rem_div(c, rk, bnd_end, bnd_begin));
     return join_side(c);
   }
-  // planes beyond LDS (FP64, no LES model): U3 and the scalars run on the
+  // the persistent kernels (FP64, no LES model): U3 and the scalars run on the
   // branch, which forks as soon as the fields are in physical space (all
   // its nonlinear pass reads), each pass on its own scratch half
   SCHK(krecord(c, 0, c.stream));  // ev_nl01
